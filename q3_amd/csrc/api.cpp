@@ -469,7 +469,7 @@ double device_bytes_held(const q3x_context_s* c, const q3x_hamiltonian_s* h) {
                                 &h->ent_pos, &h->ekin, &h->outside, &h->beta64, &h->beta32, &h->dblocks, &h->pstart,
                                 &h->psize, &h->poff, &h->zbuf, &h->P, &h->W, &h->gemm_work, &h->io_psi, &h->io_hpsi,
                                 &h->plane_slots, &h->gpack, &h->gout, &h->kb_g, &h->kb_tables, &h->kb_form,
-                                &h->kb_ints, &h->kb_dbl, &h->dens_w})
+                                &h->kb_ints, &h->kb_dbl, &h->dens_w, &h->dens_part})
             b += static_cast<double>(d->size());
         for (const FftTables& t : h->fft)
             b += static_cast<double>(t.tw64.size() + t.tw32.size() + t.plain64.size() + t.plain32.size());
@@ -1028,6 +1028,12 @@ q3x_status q3x_hamiltonian_accumulate_density(q3x_hamiltonian h, const void* d_p
         const int chunk = band_chunk(h, h->tl64, ncols);
         if (!h->zbuf.ensure(static_cast<size_t>(chunk) * h->dims[2] * h->nst * 16)) return Q3X_ERR_DEVICE;
         if (h->gamma && !h->gpack.ensure(static_cast<size_t>(h->npw_ext) * chunk * 16)) return Q3X_ERR_DEVICE;
+        const q3x_context_s* dc = h->ctx;
+        // (the last chunk may be smaller, and split into more groups)
+        for (int n : {chunk, ncols % chunk})
+            if (n > 0 && !h->dens_part.ensure(plane_density_workspace(h->dims[0], h->dims[2], h->tl64, n, dc->num_cus,
+                                                                      dc->max_lds)))
+                return Q3X_ERR_DEVICE;
         const double* psi = static_cast<const double*>(d_psi);
         for (int c0 = 0; c0 < ncols; c0 += chunk) {
             const int nc = std::min(chunk, ncols - c0);
@@ -1046,6 +1052,7 @@ q3x_status q3x_hamiltonian_accumulate_density(q3x_hamiltonian h, const void* d_p
                                                  st),
                         "density z-sticks") ||
                 !hip_ok(launch_plane_density(args, h->zbuf.as<cx<double>>(), h->tl64, nc, h->dens_w.as<double>() + 2L * c0,
+                                             h->dens_part.as<double>(), dc->num_cus, dc->max_lds,
                                              static_cast<double*>(d_rho), st),
                         "density planes"))
                 return Q3X_ERR_DEVICE;

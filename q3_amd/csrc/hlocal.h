@@ -65,9 +65,12 @@ hipError_t launch_plane_tl(const HLocalArgs& a, const T* vplane, cx<T>* zbuf, co
                            void* pglob, hipStream_t st);
 // Charge density of nvec columns of the stick buffer (after the inverse z-stick pass):
 // rho(i1, i2, i3) += wts[2c] Re(f_c(r))^2 + wts[2c+1] Im(f_c(r))^2, rho C-order (i1, i2, i3), FP64.
-// Needs the two-level plane configuration with the plane in LDS.
+// Needs the two-level plane configuration with the plane in LDS.  part: plane_density_workspace
+// bytes for the box (n = n1 = n2) and nvec, contents free.
+size_t plane_density_workspace(int n, int n3, const PlaneTlConfig& c, int nvec, int num_cus, size_t max_lds);
 hipError_t launch_plane_density(const HLocalArgs& a, const cx<double>* zbuf, const PlaneTlConfig& c, int nvec,
-                                const double* wts, double* rho, hipStream_t st);
+                                const double* wts, double* part, int num_cus, size_t max_lds, double* rho,
+                                hipStream_t st);
 // psi / hpsi: complex128, column per band with leading dimension ld (in complex elements).
 // marks (optional): 4 events recorded before/between/after the three kernels.
 // vplane: V(r)/N in plane-major layout [i3][i2][i1], double or float to match fp32.

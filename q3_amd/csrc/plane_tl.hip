@@ -79,11 +79,30 @@ __host__ __device__ constexpr int plane_tw_entries(bool fp64, int a, int b) {
 // per CU need four (128 registers); the radix-15/16 complex64 shapes need more and get two
 constexpr int plane_tl_min_waves(bool fp64, int a) { return fp64 || a > 12 ? 2 : 4; }
 
-template <typename T, int A, int B, bool PG>
+// DENS: the charge density in place of the sandwich (FP64, plane in LDS).  Workgroup (z, g) =
+// (blockIdx.x mod n3, blockIdx.x / n3) runs the backward transforms of columns [g per, g per + per)
+// of plane z and adds w_re Re(f)^2 + w_im Im(f)^2 of each into its own partial plane in dens.part,
+// which no other workgroup touches: value (row group, sub-pass, j) of a lane at
+// ((group NSR + sub-pass) B + j) 64 + lane, so a wave's 64 values are contiguous; the first column
+// stores, the others add.  density_reduce sums the groups' partials into rho.  The 96^3 box with
+// 160 columns: 6.0 -> 0.6 ms against one workgroup per (column, plane) that added every value to
+// rho atomically at a stride of n3; bound by the backward half of the sandwich's butterfly chains.
+struct PlaneDensity {
+    const double2* wts;  // (w_re, w_im) per column
+    double* part;
+    int per;             // columns per workgroup
+};
+constexpr int plane_part_size(int a, int b) {
+    const int gr = plane_group_rows(a, b);
+    return (a * b + gr - 1) / gr * ((gr * a + 63) / 64) * b * 64;
+}
+
+template <typename T, int A, int B, bool PG, bool DENS = false>
 __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
                                   plane_tl_min_waves(sizeof(T) == 8, A)) plane_tl(HLocalArgs a, const T* __restrict__ vplane,
                                                  cx<T>* __restrict__ zbuf, const cx<T>* __restrict__ twg, int lc,
-                                                 int lr, int nrw, int nplanes, cx<T>* __restrict__ pglob) {
+                                                 int lr, int nrw, int nplanes, cx<T>* __restrict__ pglob,
+                                                 PlaneDensity dens) {
     constexpr int N = A * B;
     constexpr int S = B + 1;  // stored length of a block of B slots
     constexpr int GC = plane_group_cols(sizeof(T) == 8, A, B), GR = plane_group_rows(A, B);
@@ -184,6 +203,7 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
     const int nvec = nplanes / a.p3.n;
     const bool by_xcd = (a.p3.n & 7) == 0;
     auto plane_of = [&](int q) {
+        if (DENS) return q * a.p3.n + static_cast<int>(blockIdx.x) % a.p3.n;
         if (!persist) return q;
         if (by_xcd) {
             const int j = q >> 3;
@@ -199,8 +219,12 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
             if (s < a.nst) pre[i] = src[s];
         }
     };
-    if (persist && blockIdx.x < nplanes) prefetch(plane_of(blockIdx.x));
-    for (int q = blockIdx.x; q < nplanes; q += persist ? gridDim.x : nplanes) {
+    // work items of this workgroup: planes, or with DENS the columns q of its plane
+    const int qbeg = DENS ? blockIdx.x / a.p3.n * dens.per : blockIdx.x;
+    const int qend = DENS ? min(nvec, qbeg + dens.per) : nplanes;
+    const int qstep = DENS ? 1 : persist ? gridDim.x : nplanes;
+    if (persist && qbeg < qend) prefetch(plane_of(qbeg));
+    for (int q = qbeg; q < qend; q += qstep) {
         const int plane = plane_of(q);
         const int z = plane % a.p3.n;
         for (int i = tid; i < ncol * lc; i += nt) P[i] = zero;
@@ -216,7 +240,7 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
             P[a.stick_col[s] * lc + q + q / B] = zp[s];
         }
         __syncthreads();
-        if (persist && q + static_cast<int>(gridDim.x) < nplanes) prefetch(plane_of(q + gridDim.x));
+        if (persist && q + qstep < qend) prefetch(plane_of(q + qstep));
 
         // stage 1 / stage B: lane gB * B + n2 (B lanes per transform); stage 2 / stage A: task
         // t = lane + 64 s of sub-pass s is (transform t / A, index t mod A)
@@ -256,13 +280,20 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
 
         // rows; row i2 of the plane sits at slot (i2 % A) * S + i2 / A of each column
         for (int r0 = wave * GR; wave < nrw && r0 < N; r0 += nrw * GR) {
-            // V(r) values of this lane's stage-2 tasks, loaded ahead of stage 1 so that their
-            // latency overlaps it
+            // V(r) values (DENS: partial densities) of this lane's stage-2 tasks, loaded ahead of
+            // stage 1 so that their latency overlaps it
             T vv[NSR][B];
+            double* part = nullptr;
+            if constexpr (DENS) {
+                part = dens.part + static_cast<long>(blockIdx.x) * plane_part_size(A, B) +
+                       static_cast<long>(r0 / GR) * (NSR * B * 64) + lane;
+#pragma unroll
+                for (int i = 0; i < NSR * B; ++i) vv[i / B][i % B] = q > qbeg ? part[i * 64] : 0.0;
+            }
 #pragma unroll
             for (int sp = 0; sp < NSR; ++sp) {
                 const int t = lane + 64 * sp, g = t / A, k1 = t - g * A;
-                if (g < GR && r0 + g < N) {
+                if (!DENS && g < GR && r0 + g < N) {
                     const T* vrow = vplane + (static_cast<long>(z) * N + r0 + g) * N + k1;
 #pragma unroll
                     for (int j = 0; j < B; ++j) vv[sp][j] = vrow[A * j];
@@ -295,6 +326,13 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
 #pragma unroll
                     for (int j = 0; j < B; ++j) u[j] = blk[j];
                     Dft<T, B>::run(u, T(1));
+                    if constexpr (DENS) {
+                        const double2 w = dens.wts[q];
+#pragma unroll
+                        for (int j = 0; j < B; ++j)
+                            part[(sp * B + j) * 64] = vv[sp][j] + (w.x * u[j].x * u[j].x + w.y * u[j].y * u[j].y);
+                        continue;
+                    }
 #pragma unroll
                     for (int j = 0; j < B; ++j) u[j] = cscale(u[j], vv[sp][j]);
                     Dft<T, B>::run(u, T(-1));
@@ -305,7 +343,7 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
                 }
             }
             wave_order();
-            if (gB < GR && r0 + gB < N) {  // forward stage B, lane m2; outputs i1 = m2 + B m1, occupied only
+            if (!DENS && gB < GR && r0 + gB < N) {  // forward stage B, lane m2; outputs i1 = m2 + B m1, occupied only
                 const int m2 = iB, i2 = r0 + gB;
                 const int pp = (i2 % A) * S + i2 / A;
                 const cx<T>* row = Rw + gB * lr + m2;
@@ -322,6 +360,7 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
             wave_order();
         }
         __syncthreads();
+        if constexpr (DENS) continue;
 
         // columns, forward: stage A (task n1, block n1 * S holds elements n1 + A n2), stage B
         for (int c0 = wave * GC; c0 < ncol; c0 += nw * GC) {
@@ -699,7 +738,8 @@ static hipError_t launch_one(const HLocalArgs& a, const T* vplane, cx<T>* zbuf, 
     const int nplanes = a.p3.n * nvec;
     const int grid = std::min(nplanes, std::max(1, c.workgroups));
     hipLaunchKernelGGL((plane_tl<T, A, B, PG>), dim3(grid), dim3(c.threads), c.lds, st, a, vplane, zbuf,
-                       static_cast<const cx<T>*>(a.twp), c.lc, c.lr, c.row_waves, nplanes, static_cast<cx<T>*>(pglob));
+                       static_cast<const cx<T>*>(a.twp), c.lc, c.lr, c.row_waves, nplanes, static_cast<cx<T>*>(pglob),
+                       PlaneDensity{});
     return hipGetLastError();
 }
 
@@ -753,130 +793,93 @@ template hipError_t launch_plane_tl<float>(const HLocalArgs&, const float*, cx<f
 
 // ---- charge density (PlanewaveChargeDensityAccumulator::accumulate, accumulator.hpp:77-99, and the
 // per-band |psi(r)|^2 kernel of accumulator_gpu.hpp:267 / gpu_kernels_cuda.cu:156-172), FP64.
-// Per (column, i3) plane of the stick buffer: the backward column and row transforms of
-// plane_tl, then rho(i1, i2, i3) += w_re Re(f)^2 + w_im Im(f)^2 for the real-space values f of the
-// column.  A column is one band (w_re = w_im = its weight) or, with the Gamma trick, a packed pair
-// f = f1 + i f2 of real bands (w_re, w_im = their weights).  rho is the C-order (i1, i2, i3) box;
-// the planes of different columns add into it atomically.
-template <int A, int B>
-__global__ void __launch_bounds__(512) plane_density(HLocalArgs a, const cx<double>* __restrict__ zbuf,
-                                                     const cx<double>* __restrict__ twg, int lc, int lr, int nrw,
-                                                     const double2* __restrict__ wts, double* __restrict__ rho) {
-    using T = double;
-    constexpr int N = A * B;
-    constexpr int S = B + 1;
-    constexpr int G = 64 / (A > B ? A : B);
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T>* tw = reinterpret_cast<cx<T>*>(smem_raw);
-    int* colmap = reinterpret_cast<int*>(tw + N);
-    cx<T>* P = reinterpret_cast<cx<T>*>(colmap + ((N + 3) & ~3));  // [ncol][lc]
-    const int ncol = a.ncol, n3 = a.p3.n;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
-    cx<T>* Rw = P + ncol * lc + wave * G * lr;  // this wave's [G][lr] (waves < nrw)
-    const int z = blockIdx.x, band = blockIdx.y;
-    const cx<T> zero = {T(0), T(0)};
-    for (int i = tid; i < N; i += nt) {
-        tw[i] = twg[i];
-        colmap[i] = -1;
-    }
-    for (int i = tid; i < ncol * lc; i += nt) P[i] = zero;
-    __syncthreads();
-    for (int c = tid; c < ncol; c += nt) colmap[a.col_i1[c]] = c;
-    const cx<T>* zp = zbuf + (static_cast<long>(band) * n3 + z) * a.nst;
-    for (int s = tid; s < a.nst; s += nt) {
-        const int q = a.stick_i2[s];
-        P[a.stick_col[s] * lc + q + q / B] = zp[s];
+// rho(i1, i2, i3) += w_re Re(f)^2 + w_im Im(f)^2 over the real-space values f of the columns: a
+// column is one band (w_re = w_im = its weight) or, with the Gamma trick, a packed pair f = f1 + i f2
+// of real bands (w_re, w_im = their weights).  plane_tl's DENS form leaves one partial plane per
+// (plane, column group); here they are summed in the order of the groups and added to rho, the
+// C-order (i1, i2, i3) box.  A tile of 32 partial values x 32 planes goes through LDS, so that the
+// reads run along the values and the updates of rho along i3.  The update is atomic: accumulations
+// of several contexts into one rho may overlap.
+__global__ void __launch_bounds__(256) density_reduce(int n, int a, int b, int gr, int nsr, int n3, int ngroups,
+                                                      const double* __restrict__ part, int psize,
+                                                      double* __restrict__ rho) {
+    __shared__ double tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int e0 = blockIdx.x * 32, z0 = blockIdx.y * 32;
+    for (int i = ty; i < 32; i += 8) {
+        const int z = z0 + i;
+        double s = 0.0;
+        if (z < n3)  // psize is a multiple of 64
+            for (int g = 0; g < ngroups; ++g) s += part[(static_cast<long>(g) * n3 + z) * psize + e0 + tx];
+        tile[i][tx] = s;
     }
     __syncthreads();
-    const int gB = lane / B, iB = lane - gB * B;
-    const int gA = lane / A, iA = lane - gA * A;
-    // columns, backward (as plane_tl)
-    for (int c0 = wave * G; c0 < ncol; c0 += nw * G) {
-        if (gB < G && c0 + gB < ncol) {
-            cx<T>* col = P + (c0 + gB) * lc + iB;
-            cx<T> v[A];
-#pragma unroll
-            for (int j = 0; j < A; ++j) v[j] = col[j * S];
-            Dft<T, A>::run(v, T(1));
-#pragma unroll
-            for (int k = 1; k < A; ++k) v[k] = cmulc(v[k], tw[iB * k]);
-#pragma unroll
-            for (int k = 0; k < A; ++k) col[k * S] = v[k];
-        }
-        wave_order();
-        if (gA < G && c0 + gA < ncol) {
-            cx<T>* blk = P + (c0 + gA) * lc + iA * S;
-            cx<T> u[B];
-#pragma unroll
-            for (int j = 0; j < B; ++j) u[j] = blk[j];
-            Dft<T, B>::run(u, T(1));
-#pragma unroll
-            for (int j = 0; j < B; ++j) blk[j] = u[j];
-        }
-        wave_order();
+    const int z = z0 + tx;
+    if (z >= n3) return;
+    for (int i = ty; i < 32; i += 8) {
+        const int e = e0 + i, lane = e & 63, j = (e >> 6) % b, rs = (e >> 6) / b;
+        const int t = lane + 64 * (rs % nsr), g = t / a, i1 = t - g * a + a * j, i2 = rs / nsr * gr + g;
+        if (g < gr && i2 < n) atomicAdd(rho + (static_cast<long>(i1) * n + i2) * n3 + z, tile[tx][i]);
     }
-    __syncthreads();
-    const double wr = wts[band].x, wi = wts[band].y;
-    // rows, backward, then the weighted squares; row i2 sits at slot (i2 % A) * S + i2 / A
-    for (int r0 = wave * G; wave < nrw && r0 < N; r0 += nrw * G) {
-        if (gB < G && r0 + gB < N) {
-            const int i2 = r0 + gB;
-            const int pp = (i2 % A) * S + i2 / A;
-            cx<T> v[A];
-#pragma unroll
-            for (int j = 0; j < A; ++j) {
-                const int c = colmap[B * j + iB];
-                v[j] = zero;
-                if (c >= 0) v[j] = P[c * lc + pp];
-            }
-            Dft<T, A>::run(v, T(1));
-#pragma unroll
-            for (int k = 1; k < A; ++k) v[k] = cmulc(v[k], tw[iB * k]);
-            cx<T>* row = Rw + gB * lr + iB;
-#pragma unroll
-            for (int k = 0; k < A; ++k) row[k * S] = v[k];
-        }
-        wave_order();
-        if (gA < G && r0 + gA < N) {  // lane k1: elements i1 = k1 + A j of row i2
-            const int i2 = r0 + gA;
-            const cx<T>* blk = Rw + gA * lr + iA * S;
-            cx<T> u[B];
-#pragma unroll
-            for (int j = 0; j < B; ++j) u[j] = blk[j];
-            Dft<T, B>::run(u, T(1));
-#pragma unroll
-            for (int j = 0; j < B; ++j) {
-                const long i1 = iA + A * j;
-                atomicAdd(rho + (i1 * N + i2) * n3 + z, wr * u[j].x * u[j].x + wi * u[j].y * u[j].y);
-            }
-        }
-        wave_order();
+}
+
+// Column groups per plane of a density launch: the count up to 16 whose workgroups (groups x
+// planes, `slots` of them resident at once) finish in the fewest column passes, the smaller count
+// on a tie (each group costs a partial plane).
+static int density_groups(int n3, int nvec, int slots) {
+    int best = 1;
+    long cost = std::numeric_limits<long>::max();
+    for (int g = 1; g <= std::min(nvec, 16); ++g) {
+        const int per = (nvec + g - 1) / g, used = (nvec + per - 1) / per;
+        const long c = (static_cast<long>(used) * n3 + slots - 1) / slots * per;
+        if (c < cost) cost = c, best = used;
     }
+    return best;
+}
+
+// Workgroups of the density kernel resident at once: by LDS, and two waves per SIMD by registers.
+static int density_slots(const PlaneTlConfig& c, int num_cus, size_t max_lds) {
+    return num_cus * std::max(1, std::min(static_cast<int>(max_lds / c.lds), 512 / c.threads));
+}
+
+size_t plane_density_workspace(int n, int n3, const PlaneTlConfig& c, int nvec, int num_cus, size_t max_lds) {
+    for (const TlShape& s : kTlShapes)
+        if (s.n == n)
+            return sizeof(double) * plane_part_size(s.a, s.b) * n3 *
+                   density_groups(n3, nvec, density_slots(c, num_cus, max_lds));
+    return 0;
 }
 
 template <int A, int B>
 static hipError_t launch_density_shape(const HLocalArgs& a, const cx<double>* zbuf, const PlaneTlConfig& c, int nvec,
-                                       const double* wts, double* rho, hipStream_t st) {
+                                       const double* wts, double* part, int groups, double* rho, hipStream_t st) {
     static std::atomic<bool> raised{false};
     if (!raised) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&plane_density<A, B>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&plane_tl<double, A, B, false, true>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
         raised = true;
     }
-    hipLaunchKernelGGL((plane_density<A, B>), dim3(a.p3.n, nvec), dim3(std::min(c.threads, 512)), c.lds, st, a, zbuf,
-                       static_cast<const cx<double>*>(a.twp), c.lc, c.lr, c.row_waves,
-                       reinterpret_cast<const double2*>(wts), rho);
+    const int n3 = a.p3.n, per = (nvec + groups - 1) / groups;
+    hipLaunchKernelGGL((plane_tl<double, A, B, false, true>), dim3(n3 * groups), dim3(c.threads), c.lds, st, a, nullptr,
+                       const_cast<cx<double>*>(zbuf), static_cast<const cx<double>*>(a.twp), c.lc, c.lr, c.row_waves,
+                       n3 * nvec, nullptr, PlaneDensity{reinterpret_cast<const double2*>(wts), part, per});
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    constexpr int psize = plane_part_size(A, B), gr = plane_group_rows(A, B);
+    hipLaunchKernelGGL(density_reduce, dim3(psize / 32, (n3 + 31) / 32), dim3(256), 0, st, A * B, A, B, gr,
+                       (gr * A + 63) / 64, n3, groups, part, psize, rho);
     return hipGetLastError();
 }
 
 hipError_t launch_plane_density(const HLocalArgs& a, const cx<double>* zbuf, const PlaneTlConfig& c, int nvec,
-                                const double* wts, double* rho, hipStream_t st) {
+                                const double* wts, double* part, int num_cus, size_t max_lds, double* rho,
+                                hipStream_t st) {
     if (!c.ok || c.plane_global) return hipErrorInvalidValue;
+    const int groups = density_groups(a.p3.n, nvec, density_slots(c, num_cus, max_lds));
     switch (a.p1.n) {
 #define Q3X_TL(NN, AA, BB) \
-    case NN: return launch_density_shape<AA, BB>(a, zbuf, c, nvec, wts, rho, st);
+    case NN: return launch_density_shape<AA, BB>(a, zbuf, c, nvec, wts, part, groups, rho, st);
         Q3X_TL(24, 6, 4)
         Q3X_TL(30, 6, 5)
         Q3X_TL(32, 8, 4)

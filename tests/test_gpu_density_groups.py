@@ -1,0 +1,54 @@
+"""Charge density over boxes and band counts where its split over column groups and the tiles of
+its reduction have remainders, against numpy FFTs; accumulation on top of a density."""
+import numpy as np
+import pytest
+
+from q3_amd import workloads as W
+from q3_amd.planewave import Context, DeviceArray, PlanewaveBasis, PlanewaveHamiltonianApplicator
+
+pytestmark = pytest.mark.gpu
+
+# FP64 transforms of N points err by about eps log2 N (2-norm); squares double it: 4 eps log2(1e6) = 2e-14
+TOL = 1e-13
+
+
+def _reference(basis, kp, psi, weights):
+    dims = basis.wave_dims
+    rho = np.zeros(dims)
+    for b in range(psi.shape[1]):
+        box = np.zeros(int(np.prod(dims)), np.complex128)
+        box[kp.fft_map] = psi[:, b]
+        f = np.fft.ifftn(box.reshape(dims)) * box.size
+        rho += weights[b] * np.abs(f) ** 2
+    return rho
+
+
+@pytest.mark.parametrize("kind,reps,ecut_ha,nb", [
+    ("fcc", (1, 1, 1), 15.0, 1),    # 30^3, one band: one group
+    ("fcc", (1, 1, 1), 25.0, 37),   # 36^3, odd count over several groups
+    ("sc", (1, 1, 1), 20.0, 17),    # 48^3 or the next listed size, last group short
+    ("sc", (2, 2, 1), 15.0, 5),     # n3 < n1: planes not a multiple of the 32-plane tile
+    ("sc", (2, 2, 2), 21.0, 3),     # a box of the largest radix
+])
+def test_density_groups_against_numpy(kind, reps, ecut_ha, nb):
+    c = W.alloy_cell(reps, kind, 0.0, np.random.default_rng(0))
+    basis = PlanewaveBasis(c, 2 * ecut_ha, 0.0, True, (2, 2, 2))
+    kp = basis.compute_gk([0.11, -0.23, 0.37])
+    psi = W.random_psi(kp.kinetic_energy_squared, nb, seed=nb)
+    w = np.random.default_rng(1).uniform(0.0, 2.0, nb)
+    ctx = Context(0)
+    h = PlanewaveHamiltonianApplicator(ctx, basis)
+    h.prepare_kpoint(kp)
+    ref = _reference(basis, kp, psi, w)
+    got = h.density(psi, w)
+    assert np.linalg.norm(got - ref) <= TOL * np.linalg.norm(ref)
+    # on top of a density already there, twice, and the same bits each time
+    start = np.random.default_rng(2).uniform(size=ref.size)
+    out = []
+    for _ in range(2):
+        d_psi, d_rho = DeviceArray.from_host(ctx, psi), DeviceArray.from_host(ctx, start)
+        h.accumulate_density_device(d_psi.ptr, nb, w, d_rho.ptr)
+        ctx.synchronize()
+        out.append(d_rho.download((ref.size,), np.float64))
+    assert np.array_equal(out[0], out[1])
+    assert np.linalg.norm(out[0] - start - ref.ravel()) <= 2 * TOL * np.linalg.norm(start + ref.ravel())
