@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <vector>
 
 namespace q3x {
@@ -52,15 +53,17 @@ struct Split {
 };
 
 // Upper Cholesky in place on split storage: A = U^H U.  Right-looking: after column j is
-// final, the trailing rows j of columns i > j are updated with AXPY over k.
-int chol_split(Split& A) {
+// final, the trailing rows j of columns i > j are updated with AXPY over k.  A pivot of at most
+// `rel` times its diagonal entry counts as zero.
+int chol_split(Split& A, double rel = 0.0) {
     const int n = A.n;
     for (int j = 0; j < n; ++j) {
         const double* ar = A.cr(j);
         const double* ai = A.ci(j);
-        double d = ar[j];
+        const double ajj = ar[j];
+        double d = ajj;
         for (int k = 0; k < j; ++k) d -= ar[k] * ar[k] + ai[k] * ai[k];
-        if (!(d > 0.0)) return j + 1;
+        if (!(d > rel * ajj) || !(d > 0.0)) return j + 1;
         d = std::sqrt(d);
         A.cr(j)[j] = d;
         A.ci(j)[j] = 0.0;
@@ -319,7 +322,10 @@ int chol_upper(int n, zc* A, int lda) {
             S.cr(j)[i] = A[ix(i, j, lda)].real();
             S.ci(j)[i] = A[ix(i, j, lda)].imag();
         }
-    const int info = chol_split(S);
+    // a pivot within the rounding of its own computation (n eps, the rank test of LAPACK's pivoted
+    // Cholesky) has no digits left: a block with repeated columns must not pass as positive definite
+    // because its zero pivot happened to round up
+    const int info = chol_split(S, n * std::numeric_limits<double>::epsilon());
     if (info) return info;
     for (int j = 0; j < n; ++j)
         for (int i = 0; i < n; ++i) A[ix(i, j, lda)] = (i <= j) ? zc(S.cr(j)[i], S.ci(j)[i]) : zc(0, 0);

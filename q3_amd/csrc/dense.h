@@ -6,7 +6,8 @@ namespace q3x {
 
 using zc = std::complex<double>;
 
-// A = U^H U (upper).  Returns 0, or j+1 if the leading minor j+1 is not positive definite.
+// A = U^H U (upper).  Returns 0, or j+1 if the leading minor j+1 is not positive definite to
+// rounding (pivot <= n eps A_jj).
 int chol_upper(int n, zc* A, int lda);
 // U <- U^{-1} for upper-triangular U (lower part ignored and zeroed).
 void tri_inv_upper(int n, zc* U, int ldu);
