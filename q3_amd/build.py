@@ -29,7 +29,7 @@ EXTRA = {
                   "-fno-math-errno"],
     "davidson.cpp": ["-fopenmp"],
 }
-SOURCES = ["setup.cpp", "kb_projectors.cpp", "api.cpp", "hlocal.hip", "plane_tl.hip", "zgemm.hip", "aux_kernels.hip",
+SOURCES = ["setup.cpp", "kb_projectors.cpp", "api.cpp", "hlocal.hip", "plane_tl.hip", "zgemm.hip", "zgemm64.hip", "aux_kernels.hip",
            "subspace_eig.hip", "potential.hip", "noalloc.hip", "gamma_kernels.hip", "kb_device.hip", "dense.cpp", "davidson.cpp", "batch.cpp", "server.cpp",
            "memory_estimate.cpp"]
 

@@ -15,4 +15,12 @@ hipError_t zgemm(GemmTypes types, int opa, int m, int n, int k, double alpha, co
                  const void* B, long ldb, double beta, void* C, long ldc, void* work, size_t work_bytes,
                  hipStream_t st);
 
+// The FP64 products (zgemm64.hip) of 16-byte aligned matrices: m, n > 0.  tile: 10 r + c for a
+// workgroup tile of 32 r rows by 16 c complex columns (44, 42, 25, 24, 23, 22, 21, 12) or 0 for the
+// built-in choice; split: K chunks, <= 0 for the built-in choice.
+bool zgemm64_has_tile(int tile);
+bool zgemm64_aligned(const void* A, const void* B, const void* C, const void* work);
+hipError_t zgemm64(int tile, int split, int opa, int m, int n, int k, double alpha, const void* A, long lda, const void* B,
+                   long ldb, double beta, void* C, long ldc, void* work, size_t work_bytes, hipStream_t st);
+
 }  // namespace q3x

@@ -1,4 +1,6 @@
-// Complex GEMM on CDNA4 matrix cores (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32).
+// Complex GEMM on CDNA4 matrix cores with register-staged operands (v_mfma_f32_16x16x4f32, and
+// v_mfma_f64_16x16x4f64 for FP64 matrices that are not 16-byte aligned; the aligned ones go to
+// zgemm64.hip).
 //
 //   C (m x n) = alpha * op(A) * B + beta * C,   op(A) = A (m x k) or A^H (A stored k x m),
 //   alpha, beta real, all matrices column-major interleaved complex.
@@ -72,10 +74,8 @@ __global__ void __launch_bounds__(256, MINW) zgemm_kernel(int m, int n, int k, i
     constexpr int NLB = (BNC * KC + 255) / 256;  // B loads per thread per stage
     __shared__ TM As[2][2 * KC * LA];
     // FP64 (BC): B stored once per k, row p = [Br Bi Br Bi ...]; row 2p of B' is row p and row
-    // 2p + 1 is row p with each (Br, Bi) pair read swapped and its real part negated.  Half the
-    // LDS of B' (the 2x5 tiles reach three workgroups per CU instead of two): cfg2 projector
-    // overlap 0.373 -> 0.349 ms, update 0.360 -> 0.340 ms.  Complex64 keeps B' expanded (its
-    // overlap ran 5% slower with the compact form)
+    // 2p + 1 is row p with each (Br, Bi) pair read swapped and its real part negated, which halves
+    // the LDS of B'.  Complex64 keeps B' expanded (its overlap ran 5% slower with the compact form)
     constexpr bool BC = sizeof(TM) == 8;
     __shared__ TM Bs[2][(BC ? 1 : 2) * KC * LB];
     const int tid = threadIdx.x;
@@ -301,10 +301,8 @@ hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A
         ksplit = static_cast<int>(std::max(1L, std::min(want, std::min(by_k, by_ws))));
     }
     // FP64: split K over a multiple of 8 chunks when there are 8 or more, so that each chunk's
-    // tiles share one XCD (xmap in zgemm_kernel).  At cfg2 the projector overlap then reads 347 MB
-    // (the algorithmic 343 MB) instead of 977 MB in the same time: the kernel is not bound by
-    // HBM, and the traffic saved is left to concurrent work.  The complex64 products ran 4% slower
-    // with it (1% with the chunk count kept a multiple of 8: 0.228 vs 0.225 ms for the cfg2
+    // tiles share one XCD (xmap in zgemm_kernel).  The complex64 products ran 4% slower with it (1%
+    // with the chunk count kept a multiple of 8: 0.228 vs 0.225 ms for the 256 x 160 x 51,627
     // overlap) and keep the plain order.
     // The chunk count stays that multiple of 8 after the chunk length is rounded up to KC: chunks
     // past the end of K are empty and add zero partials.
@@ -318,9 +316,8 @@ hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A
     int xmap = want_xmap && ksplit % 8 == 0 ? 1 : 0;
     dim3 grid(tm, tn, ksplit);
     // A B without a split (the projector update Hpsi += beta W): the column tiles of a row block
-    // run one after another on one XCD (xmap 2), so each row block of A is fetched once: at cfg2
-    // the FP64 update reads 392 MB instead of 1,270 MB (0.365 -> 0.360 ms), complex64 286 instead
-    // of 802 MB in the same time
+    // run one after another on one XCD (xmap 2), so each row block of A is fetched once: the
+    // complex64 update of 51,627 x 160 x 256 reads 286 MB instead of 802 MB in the same time
     if (opa == 0 && ksplit == 1 && tn > 1) {
         xmap = 2;
         grid.x = (tm + 7) / 8 * 8;
@@ -342,12 +339,11 @@ hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A
     return hipGetLastError();
 }
 
-// Tile configurations (wave tiles TMW x TNW, K stage KC, minimum waves per SIMD) and how a
+// Tile configurations (wave tiles TMW x TNW, K stage KC, minimum waves per SIMD) and how a complex64
 // product picks one.  The table comes from timing every candidate on the H|psi> and Davidson
-// shapes of the 64-atom cell (q3_amd/tune_gemm.py).  Deep-k A^H B products split K so that
-// the grid is one round of resident workgroups (CUs x occupancy of the kernel): a partial
-// second round costs as much as a full one.  FP64 A^H B: 2x5 tiles when n fills 80-column
-// tiles, else 2x2; FP64 A B (tall m): 4x2 tiles at two waves per SIMD; FP32: 2x2 tiles.
+// shapes of the 64-atom cell (q3_amd/tune_gemm.py): 2x2 tiles throughout; deep-k A^H B products
+// split K so that the grid is one round of resident workgroups (CUs x occupancy of the kernel): a
+// partial second round costs as much as a full one.
 // Q3X_GEMM_TILE="TMWxTNW/ksplit" overrides the choice (ksplit -1: one round, 0: default).
 enum class Tile { T2x2, T4x2, T2x5, T4x4, T4x5 };
 
@@ -379,25 +375,29 @@ template <typename TA, typename TB, typename TM, typename TC>
 hipError_t zgemm_t(int opa, int m, int n, int k, double alpha, const void* A, long lda, const void* B, long ldb,
                    double beta, void* C, long ldc, void* work, size_t work_bytes, hipStream_t st) {
     if (m <= 0 || n <= 0) return hipSuccess;
-    if (const char* cfg = std::getenv("Q3X_GEMM_TILE")) {
-        int tmw = 0, tnw = 0, sp = 0;
-        if (std::sscanf(cfg, "%dx%d/%d", &tmw, &tnw, &sp) == 3) {  // sp: -1 one round, 0 default, > 0 fixed
-            const Tile t = tmw == 4 ? (tnw == 2 ? Tile::T4x2 : tnw == 4 ? Tile::T4x4 : Tile::T4x5)
-                                    : (tnw == 5 ? Tile::T2x5 : Tile::T2x2);
-            return zgemm_tile<TA, TB, TM, TC>(t, sp, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                              work_bytes, st);
+    if constexpr (std::is_same<TM, double>::value) {
+        if (zgemm64_aligned(A, B, C, work)) {
+            int tmw = 0, tnw = 0, sp = 0, tile = 0;
+            const char* cfg = std::getenv("Q3X_GEMM_TILE");
+            if (cfg && std::sscanf(cfg, "%dx%d/%d", &tmw, &tnw, &sp) == 3) tile = 10 * tmw + tnw;
+            if (!zgemm64_has_tile(tile)) tile = sp = 0;
+            return zgemm64(tile, sp, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, st);
         }
+        return zgemm_shape<TA, TB, TM, TC, 2, 2, 8, 1>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+                                                       work_bytes, st, opa == 1 ? -1 : 0);
+    } else {
+        if (const char* cfg = std::getenv("Q3X_GEMM_TILE")) {
+            int tmw = 0, tnw = 0, sp = 0;
+            if (std::sscanf(cfg, "%dx%d/%d", &tmw, &tnw, &sp) == 3) {  // sp: -1 one round, 0 default, > 0 fixed
+                const Tile t = tmw == 4 ? (tnw == 2 ? Tile::T4x2 : tnw == 4 ? Tile::T4x4 : Tile::T4x5)
+                                        : (tnw == 5 ? Tile::T2x5 : Tile::T2x2);
+                return zgemm_tile<TA, TB, TM, TC>(t, sp, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+                                                  work_bytes, st);
+            }
+        }
+        return zgemm_tile<TA, TB, TM, TC>(Tile::T2x2, opa == 1 ? -1 : 0, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+                                          work_bytes, st);
     }
-    const bool f64 = std::is_same<TM, double>::value;
-    Tile t = Tile::T2x2;
-    if (m > 64 && n > 32) {
-        if (opa == 1)
-            t = f64 && n % 80 == 0 ? Tile::T2x5 : Tile::T2x2;
-        else
-            t = f64 ? Tile::T4x2 : Tile::T2x2;
-    }
-    return zgemm_tile<TA, TB, TM, TC>(t, opa == 1 ? -1 : 0, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                      work_bytes, st);
 }
 
 }  // namespace

@@ -1,10 +1,10 @@
 """Tile tuner for the complex MFMA GEMM (zgemm.hip).
 
-Times every wave-tile configuration the library is built with (and a few K splits for the
-deep-k A^H B products) on the products of H|psi> and block Davidson for a given plane-wave
+Times every tile configuration the library is built with (and a few K splits for the deep-k A^H B
+products; a tile TMWxTNW covers 32 TMW rows and 16 TNW complex columns per workgroup) on the products of H|psi> and block Davidson for a given plane-wave
 count, band count and projector count, and prints the fastest per shape class and precision.
-The library's built-in table (zgemm.hip, zgemm_t) is what this printed for the 64-atom Si cell
-(npw 51,627, 160 bands, 256 projectors); Q3X_GEMM_TILE="TMWxTNW/ksplit" forces one
+The library's built-in choices (the cost model of zgemm64.hip, the complex64 table of zgemm.hip)
+were fitted to what this printed for the 64-atom Si cell (npw 51,627, 160 bands, 256 projectors); Q3X_GEMM_TILE="TMWxTNW/ksplit" forces one
 configuration at run time, which is how this script measures the candidates.
 
     python -m q3_amd.tune_gemm [--npw 51627] [--bands 160] [--nproj 256] [--reps 20]
@@ -18,7 +18,8 @@ import time
 
 import numpy as np
 
-TILES = ["2x2", "4x2", "2x5", "4x4", "4x5"]
+TILES = {"fp64": ["4x4", "4x2", "2x5", "2x4", "2x3", "2x2", "2x1", "1x2"],  # zgemm64.hip
+         "fp32": ["2x2", "4x2", "2x5", "4x4", "4x5"]}                          # zgemm.hip
 SPLITS = [-1, 0, 64, 128]
 
 
@@ -51,7 +52,7 @@ def main(argv=None):
         lda = m if ta == "N" else k
         flops = 8.0 * m * n * k
         for prec, label in ((FP64, "fp64"), (MIXED, "fp32")):
-            cands = [("", None)] + [(f"{t}/{s}", t) for t in TILES for s in (SPLITS if ta == "C" else [0])]
+            cands = [("", None)] + [(f"{t}/{s}", t) for t in TILES[label] for s in (SPLITS if ta == "C" else [0])]
             best = None
             for cfg, _ in cands:
                 if cfg:
