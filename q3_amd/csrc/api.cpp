@@ -206,14 +206,14 @@ bool build_tables(FftTables& t, int n, hipStream_t st, HostStage* pin) {
 
 HLocalArgs make_args(const q3x_hamiltonian_s* h, bool fp32) {
     HLocalArgs a{};
-    a.p1 = h->fft[0].plan;
-    a.p2 = h->fft[1].plan;
-    a.p3 = h->fft[2].plan;
-    a.tw1 = fp32 ? h->fft[0].tw32.get() : h->fft[0].tw64.get();
-    a.tw2 = fp32 ? h->fft[1].tw32.get() : h->fft[1].tw64.get();
-    a.tw3 = fp32 ? h->fft[2].tw32.get() : h->fft[2].tw64.get();
-    a.twp = fp32 ? h->fft[0].plain32.get() : h->fft[0].plain64.get();
-    a.twp3 = fp32 ? h->fft[2].plain32.get() : h->fft[2].plain64.get();
+    a.p1 = h->fft[h->axis[0]].plan;
+    a.p2 = h->fft[h->axis[1]].plan;
+    a.p3 = h->fft[h->axis[2]].plan;
+    a.tw1 = fp32 ? h->fft[h->axis[0]].tw32.get() : h->fft[h->axis[0]].tw64.get();
+    a.tw2 = fp32 ? h->fft[h->axis[1]].tw32.get() : h->fft[h->axis[1]].tw64.get();
+    a.tw3 = fp32 ? h->fft[h->axis[2]].tw32.get() : h->fft[h->axis[2]].tw64.get();
+    a.twp = fp32 ? h->fft[h->axis[0]].plain32.get() : h->fft[h->axis[0]].plain64.get();
+    a.twp3 = fp32 ? h->fft[h->axis[2]].plain32.get() : h->fft[h->axis[2]].plain64.get();
     a.nst = h->nst;
     a.ncol = h->ncol;
     a.sticks_per_block = h->sticks_per_block;
@@ -232,8 +232,8 @@ HLocalArgs make_args(const q3x_hamiltonian_s* h, bool fp32) {
 
 // Largest band chunk whose stick buffer (and plane slots, for planes kept outside LDS) stays under 2 GiB.
 int band_chunk(const q3x_hamiltonian_s* h, const PlaneTlConfig& tl, int nvec) {
-    size_t per = static_cast<size_t>(h->dims[2]) * h->nst * 16;
-    if (tl.ok && tl.plane_global) per += static_cast<size_t>(h->dims[2]) * tl.plane_bytes;
+    size_t per = static_cast<size_t>(h->n3()) * h->nst * 16;
+    if (tl.ok && tl.plane_global) per += static_cast<size_t>(h->n3()) * tl.plane_bytes;
     const size_t cap = size_t(2) << 30;
     int c = static_cast<int>(std::max<size_t>(1, cap / std::max<size_t>(per, 1)));
     return std::min(c, nvec);
@@ -264,8 +264,8 @@ q3x_status hamiltonian_apply_device(q3x_hamiltonian h, const double* d_psi, long
     const int nvec_t = h->gamma ? (nvec + 1) / 2 : nvec;
     const int chunk = band_chunk(h, tl, nvec_t);
     const size_t cs = fp32 ? 8 : 16;
-    if (!h->zbuf.ensure(static_cast<size_t>(chunk) * h->dims[2] * h->nst * cs)) return Q3X_ERR_DEVICE;
-    if (tl.ok && tl.plane_global && !h->plane_slots.ensure(static_cast<size_t>(chunk) * h->dims[2] * tl.plane_bytes))
+    if (!h->zbuf.ensure(static_cast<size_t>(chunk) * h->n3() * h->nst * cs)) return Q3X_ERR_DEVICE;
+    if (tl.ok && tl.plane_global && !h->plane_slots.ensure(static_cast<size_t>(chunk) * h->n3() * tl.plane_bytes))
         return Q3X_ERR_DEVICE;
     const void* vplane = fp32 ? h->v32.get() : h->v64.get();
     Profiler& pr = h->ctx->prof;
@@ -360,8 +360,8 @@ size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 // Scratch bytes of one band chunk of nb bands carved from a fixed region: stick buffer, plane
 // slots (planes kept outside LDS), P and W of the projector chain, each 256-byte aligned.
 size_t fixed_chunk_bytes(const q3x_hamiltonian_s* h, const PlaneTlConfig& tl, int nb, size_t cs) {
-    size_t b = align256(static_cast<size_t>(nb) * h->dims[2] * h->nst * cs);
-    if (tl.ok && tl.plane_global) b += align256(static_cast<size_t>(nb) * h->dims[2] * tl.plane_bytes);
+    size_t b = align256(static_cast<size_t>(nb) * h->n3() * h->nst * cs);
+    if (tl.ok && tl.plane_global) b += align256(static_cast<size_t>(nb) * h->n3() * tl.plane_bytes);
     if (h->have_projectors && h->nproj > 0) b += 2 * align256(static_cast<size_t>(h->nproj) * nb * cs);
     return b;
 }
@@ -407,8 +407,8 @@ q3x_status hamiltonian_apply_fixed(q3x_hamiltonian h, const double* d_psi, doubl
     // largest chunk of bands whose buffers fit, leaving the split-K workspace the rest
     int chunk = static_cast<int>(std::min<size_t>(static_cast<size_t>(nvec), scratch_bytes / one));
     while (chunk > 1 && fixed_chunk_bytes(h, tl, chunk, cs) > scratch_bytes) --chunk;
-    const size_t zb = align256(static_cast<size_t>(chunk) * h->dims[2] * h->nst * cs);
-    const size_t sb = tl.ok && tl.plane_global ? align256(static_cast<size_t>(chunk) * h->dims[2] * tl.plane_bytes) : 0;
+    const size_t zb = align256(static_cast<size_t>(chunk) * h->n3() * h->nst * cs);
+    const size_t sb = tl.ok && tl.plane_global ? align256(static_cast<size_t>(chunk) * h->n3() * tl.plane_bytes) : 0;
     const bool nonlocal = h->have_projectors && h->nproj > 0;
     const size_t pb = nonlocal ? align256(static_cast<size_t>(h->nproj) * chunk * cs) : 0;
     char* zbuf = scratch;
@@ -488,6 +488,7 @@ q3x_status hamiltonian_rebind(q3x_hamiltonian h, q3x_basis b) {
                            h->fft[2].plan.n == b->d.wave[2] && h->fft[0].plain64.size() > 0;
     h->basis = b;
     for (int d = 0; d < 3; ++d) h->dims[d] = b->d.wave[d];
+    transform_axes(h->dims, h->axis);
     h->npoints = static_cast<long>(h->dims[0]) * h->dims[1] * h->dims[2];
     h->have_potential = false;
     h->kp = nullptr;
@@ -816,14 +817,17 @@ q3x_status q3x_hamiltonian_set_potential(q3x_hamiltonian h, const double* v, lon
                 return Q3X_ERR_DEVICE;
             vs = restricted.data();
         }
-        const int n1 = h->dims[0], n2 = h->dims[1], n3 = h->dims[2];
+        // plane-major along the transforms' axes: [i3][i2][i1]
+        const long stride[3] = {static_cast<long>(h->dims[1]) * h->dims[2], h->dims[2], 1};
+        const long s1 = stride[h->axis[0]], s2 = stride[h->axis[1]], s3 = stride[h->axis[2]];
+        const int n1 = h->dims[h->axis[0]], n2 = h->dims[h->axis[1]], n3 = h->n3();
         const double inv = 1.0 / static_cast<double>(h->npoints);  // serial.hpp:69-73
         std::vector<double> d(h->npoints);
         std::vector<float> f(h->npoints);
         for (int i1 = 0; i1 < n1; ++i1)
             for (int i2 = 0; i2 < n2; ++i2)
                 for (int i3 = 0; i3 < n3; ++i3) {
-                    const double s = vs[(static_cast<long>(i1) * n2 + i2) * n3 + i3] * inv;
+                    const double s = vs[i1 * s1 + i2 * s2 + i3 * s3] * inv;
                     const long o = (static_cast<long>(i3) * n2 + i2) * n1 + i1;
                     d[o] = s;
                     f[o] = static_cast<float>(s);
@@ -860,7 +864,7 @@ q3x_status q3x_hamiltonian_prepare_kpoint(q3x_hamiltonian h, q3x_kpoint k) {
         for (int p = 0; p < h->npw_ext; ++p)
             if (tmap[p] < 0) out.push_back(p);
         h->n_outside = static_cast<int>(out.size());
-        const int n1 = h->dims[0], n2 = h->dims[1], n3 = h->dims[2];
+        const int n1 = h->dims[h->axis[0]], n2 = h->dims[h->axis[1]], n3 = h->n3();
         h->sticks_per_block = std::max(4, std::min(64, 3072 / n3));
         // two-level plane kernel where the plane is square and of a size it is built for;
         // Q3X_FFT_KERNELS=generic keeps the Stockham kernels (used to compare the two)
@@ -1005,7 +1009,8 @@ q3x_status q3x_hamiltonian_accumulate_density(q3x_hamiltonian h, const void* d_p
             set_error("q3x_hamiltonian_accumulate_density: prepare_kpoint() must come first");
             return Q3X_ERR_STATE;
         }
-        if (!h->tl64.ok || h->tl64.plane_global || !h->tz64.ok || h->n_outside > 0) {
+        // rho is laid out along the box axes, so the planes must be the box's own (n1 = n2)
+        if (!h->tl64.ok || h->tl64.plane_global || !h->tz64.ok || h->n_outside > 0 || h->axis[2] != 2) {
             set_error("q3x_hamiltonian_accumulate_density: the wavefunction box must be one the two-level kernels "
                       "cover (square planes of a listed size, the plane in LDS) and hold every plane wave");
             return Q3X_ERR_ARGUMENT;
@@ -1026,12 +1031,12 @@ q3x_status q3x_hamiltonian_accumulate_density(q3x_hamiltonian h, const void* d_p
         }
         if (!h->dens_w.upload(w2.data(), w2.size() * sizeof(double), st, &h->ctx->pin)) return Q3X_ERR_DEVICE;
         const int chunk = band_chunk(h, h->tl64, ncols);
-        if (!h->zbuf.ensure(static_cast<size_t>(chunk) * h->dims[2] * h->nst * 16)) return Q3X_ERR_DEVICE;
+        if (!h->zbuf.ensure(static_cast<size_t>(chunk) * h->n3() * h->nst * 16)) return Q3X_ERR_DEVICE;
         if (h->gamma && !h->gpack.ensure(static_cast<size_t>(h->npw_ext) * chunk * 16)) return Q3X_ERR_DEVICE;
         const q3x_context_s* dc = h->ctx;
         // (the last chunk may be smaller, and split into more groups)
         for (int n : {chunk, ncols % chunk})
-            if (n > 0 && !h->dens_part.ensure(plane_density_workspace(h->dims[0], h->dims[2], h->tl64, n, dc->num_cus,
+            if (n > 0 && !h->dens_part.ensure(plane_density_workspace(h->dims[0], h->n3(), h->tl64, n, dc->num_cus,
                                                                       dc->max_lds)))
                 return Q3X_ERR_DEVICE;
         const double* psi = static_cast<const double*>(d_psi);

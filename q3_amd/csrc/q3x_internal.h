@@ -44,6 +44,14 @@ struct BasisData {
     std::vector<GEntry> g;
 };
 
+// Box axes of the transforms: axis[0] along the rows of a plane, axis[1] along its columns, axis[2]
+// along the sticks.  (0, 1, 2), or where n1 != n2 and two axes are of one length that the two-level
+// plane kernels are built for, the order that puts those two into the plane: a 72 x 36 x 36 box runs
+// its square 36 x 36 planes there instead of 72 x 36 planes in the generic kernel (75 x 40 x 40, 39
+// bands: plane stage 188 -> 63 us).  Lengths up to 120, whose planes the generic kernels can hold in
+// LDS too.  i1, i2, i3 below and in the kernels count along axis[0], axis[1], axis[2].
+void transform_axes(const int wave[3], int axis[3]);
+
 // Stick decomposition of one k-point's sphere for the pencil FFT.
 //   sticks: distinct (m1, m2) pairs, ordered by (column, i2); column = rank of wrapped i1.
 //   entries: one per plane wave, stick-major, z ascending within a stick.

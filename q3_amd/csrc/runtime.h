@@ -116,6 +116,8 @@ struct q3x_hamiltonian_s {
     q3x_context ctx = nullptr;
     const q3x_basis_s* basis = nullptr;
     int dims[3] = {0, 0, 0};
+    int axis[3] = {0, 1, 2};  // box axes of the transforms (transform_axes)
+    int n3() const { return dims[axis[2]]; }  // length of a stick, number of planes
     long npoints = 0;
     q3x::FftTables fft[3];
     // potential V(r)/N, plane-major [i3][i2][i1]

@@ -13,6 +13,7 @@
 #include <numeric>
 #include <stdexcept>
 
+#include "hlocal.h"
 #include "q3x_internal.h"
 
 namespace q3x {
@@ -119,19 +120,30 @@ static void build_sphere(BasisData& B) {
 
 static int wrap(int m, int n) { return m >= 0 ? m : m + n; }
 
+void transform_axes(const int wave[3], int axis[3]) {
+    const int n1 = wave[0], n2 = wave[1], n3 = wave[2];
+    auto square = [](int n) { return n <= 120 && plane_tl_supported(n, n); };
+    const bool swap3 = n1 != n2 && (n2 == n3 || n1 == n3) && square(n3);
+    axis[0] = swap3 && n2 == n3 ? 1 : 0;
+    axis[1] = swap3 ? 2 : 1;
+    axis[2] = !swap3 ? 2 : n2 == n3 ? 0 : 1;
+}
+
 // Stick layout for the pencil FFT.  Permutation-only bookkeeping: values are never reordered
 // in HBM, the kernels gather/scatter through ent_pw.
 // millers: 3 ints per plane wave of the list the transforms run over; fftmap: its box offsets
 // (-1 outside the box).
 static void build_sticks(const int wave[3], const std::vector<int>& millers, const std::vector<int>& fftmap,
                          StickLayout& S) {
-    const int n1 = wave[0], n2 = wave[1], n3 = wave[2];
+    int ax[3];
+    transform_axes(wave, ax);
+    const int n1 = wave[ax[0]], n2 = wave[ax[1]], n3 = wave[ax[2]];
     const int npw = static_cast<int>(fftmap.size());
     // distinct columns (wrapped i1) present
     std::vector<char> has_col(n1, 0);
     for (int p = 0; p < npw; ++p) {
         if (fftmap[p] < 0) continue;
-        has_col[wrap(millers[3 * p], n1)] = 1;
+        has_col[wrap(millers[3 * p + ax[0]], n1)] = 1;
     }
     std::vector<int> col_of_i1(n1, -1);
     S.col_i1.clear();
@@ -147,11 +159,11 @@ static void build_sticks(const int wave[3], const std::vector<int>& millers, con
     for (int p = 0; p < npw; ++p) {
         if (fftmap[p] < 0) continue;
         const int* m = &millers[3 * p];
-        int c = col_of_i1[wrap(m[0], n1)];
-        int key = c * n2 + wrap(m[1], n2);
+        int c = col_of_i1[wrap(m[ax[0]], n1)];
+        int key = c * n2 + wrap(m[ax[1]], n2);
         stick_id[key] = 0;
         pw_stick[p] = key;
-        pw_z[p] = wrap(m[2], n3);
+        pw_z[p] = wrap(m[ax[2]], n3);
     }
     S.stick_col.clear();
     S.stick_i2.clear();
