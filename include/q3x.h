@@ -235,7 +235,7 @@ q3x_status q3x_hegv(int n, const double* H, const double* S, double* w, double* 
 q3x_status q3x_hegv_device(q3x_context ctx, int n, const void* H, long ldh, const void* S, long lds,
                            int nvec, double* w, void* X, long ldx);
 /* No counterpart in the reference.  Test hook of the device eigensolver: the next `count`
- * multi-workgroup tridiagonalisations (n >= 100) start with their grid-barrier give-up flag set,
+ * multi-workgroup tridiagonalisations (n > 128) start with their grid-barrier give-up flag set,
  * so each runs to its end without waiting and its solve is redone on one workgroup, as when
  * another stream's work keeps a workgroup from being placed. */
 void q3x_debug_force_barrier_giveups(int count);

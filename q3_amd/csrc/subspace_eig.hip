@@ -9,10 +9,10 @@
 //      not positive definite, which is reported as zhegv's info > n.
 //   2. C = Z H Z (two GEMMs).  The eigenvectors of the pencil are X = Z Y with C Y = Y w, and
 //      X^H S X = I.
-//   3. C = Q T Q^H by Householder reflectors in one workgroup: the rank-2 update of step k and
+//   3. C = Q T Q^H by Householder reflectors: the rank-2 update of step k and
 //      the matrix-vector product of step k+1 share one pass over the trailing block (look-
-//      ahead on the next column), so each step reads and writes the block once.  For n <= 99
-//      the matrix sits in LDS.
+//      ahead on the next column), so each step touches the block once.  Up to n = 512 the matrix
+//      stays in registers, of one CU (n <= 128) or of several.
 //   4. T = D Tr D^H with a real tridiagonal Tr (phases D); eigenvalues of Tr by multisection:
 //      one wavefront per eigenvalue, 63 Sturm counts per round, 6 bits per round.
 //   5. Eigenvectors of Tr, one thread per vector, in parallel: an isolated eigenvalue by one
@@ -84,18 +84,37 @@ __device__ __forceinline__ double wave_sum(double v) {
 // stage swaps half of the live values with the partner lane and adds, halving V, so V sums
 // cost about log2(64) + V - 1 exchanges instead of 6 V.  On return lane l holds the full sum of
 // value l / (64 / V).
-// Orders a wavefront's LDS accesses across lanes (they execute in issue order; this keeps the
-// compiler from moving them across the point).
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+// Sum of two values over lane pairs l, l ^ 32 (SWAP32) or l ^ 16: the lanes with that bit clear get
+// the sum of a, the others that of b.  A lane swap between the two registers leaves both addends of a
+// lane's sum in that lane, without selects and without an LDS round trip.
+template <bool SWAP32>
+__device__ __forceinline__ double swap_sum(double a, double b) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    u2 lo, hi;
+    if (SWAP32) {
+        lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+        hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    } else {
+        lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+        hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    }
+    return __hiloint2double(static_cast<int>(hi.x), static_cast<int>(lo.x)) +
+           __hiloint2double(static_cast<int>(hi.y), static_cast<int>(lo.y));
 }
 
 template <int V>
 __device__ __forceinline__ double wave_multi_sum(double (&x)[V], int lane) {
-    int o = 32;
+    static_assert(V >= 2 && V <= 32, "at least one value to swap");
 #pragma unroll
-    for (int h = V / 2; h >= 1; h /= 2, o /= 2) {
+    for (int i = 0; i < V / 2; ++i) x[i] = swap_sum<true>(x[i], x[i + V / 2]);
+#pragma unroll
+    for (int i = 0; i < V / 4; ++i) x[i] = swap_sum<false>(x[i], x[i + V / 4]);
+    if (V == 2) x[0] = swap_sum<false>(x[0], x[0]);
+    // within a row of 16: the exchange partner by DPP moves that flip the stage's lane bit (row mirror,
+    // half-row mirror, quad permutes; the lower bits they flip too are summed over later)
+    int o = 8;
+#pragma unroll
+    for (int h = V / 8; h >= 1; h /= 2, o /= 2) {
         const bool up = (lane & o) != 0;
 #pragma unroll
         for (int i = 0; i < h; ++i) {
@@ -103,23 +122,24 @@ __device__ __forceinline__ double wave_multi_sum(double (&x)[V], int lane) {
             // otherwise folded into one load at a lane-dependent index, which moves x to scratch
             double lo = x[i], hi = x[i + h];
             asm volatile("" : "+v"(lo), "+v"(hi));
-            const double send = up ? lo : hi;
-            const double keep = up ? hi : lo;
-            x[i] = keep + __shfl_xor(send, o, 64);
+            const double send = up ? lo : hi, keep = up ? hi : lo;
+            x[i] = keep + (o == 8 ? dpp_mov<0x140>(send) : o == 4 ? dpp_mov<0x141>(send) : dpp_mov<0x4E>(send));
         }
     }
-    // the remaining plain sums: across rows by shuffles, within a row of 16 by DPP moves (row
-    // mirror, half-row mirror, quad permutes: each pairs the lanes of the group still to be
-    // summed, in the VALU, without an LDS round trip)
     double s = x[0];
-#pragma unroll
-    for (; o >= 16; o /= 2) s += __shfl_xor(s, o, 64);
     if (o >= 8) s += dpp_mov<0x140>(s);
     if (o >= 4) s += dpp_mov<0x141>(s);
     if (o >= 2) s += dpp_mov<0x4E>(s);
     if (o >= 1) s += dpp_mov<0xB1>(s);
     return s;
 }
+// Orders a wavefront's LDS accesses across lanes (they execute in issue order; this keeps the
+// compiler from moving them across the point).
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
@@ -242,6 +262,65 @@ __global__ void scale_matrix(long nn, double s, z2* __restrict__ A) {
 }
 
 // ---------------------------------------------------------------- 3. tridiagonalisation ----
+// 1 / sqrt(x) to about an ulp for normal x > 0 (hardware estimate and two Newton steps).
+__device__ __forceinline__ double rsqrt_ulp(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+    r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+    return r;
+}
+
+// Reflector scalars of (x0, tail), tail = sum |x_i|^2 of the rest > 0: H^H x = b e_0,
+// w_i = x_i s below the leading 1, and tau = 2 / (1 + sum |w|^2) = 1 + |x0| / |x|.
+struct Reflector {
+    z2 b, s;
+    double tau;
+};
+__device__ __forceinline__ Reflector reflector(z2 x0, double tail) {
+    const double a2 = x0.x * x0.x + x0.y * x0.y, nn = tail + a2;
+    double a0, xn, ixn;
+    z2 ph;
+    if (a2 > 1e-280 && nn < 1e280) {
+        const double ra = rsqrt_ulp(a2);
+        ixn = rsqrt_ulp(nn);
+        a0 = a2 * ra;
+        xn = nn * ixn;
+        ph = {x0.x * ra, x0.y * ra};
+    } else {
+        a0 = hypot(x0.x, x0.y);
+        xn = sqrt(tail + a0 * a0);
+        ixn = 1.0 / xn;
+        ph = a0 == 0.0 ? z2{1.0, 0.0} : z2{x0.x / a0, x0.y / a0};
+    }
+    const double iu = div_ulp(1.0, a0 + xn);  // u0 = x0 - b = ph (a0 + xn)
+    return {{-ph.x * xn, -ph.y * xn}, {ph.x * iu, -ph.y * iu}, 1.0 + a0 * ixn};
+}
+
+// T = D Tr D^H: |beta| into eabs and the running product of the phases of beta into phase, by one
+// wavefront: each lane multiplies a run of consecutive entries, the runs are scanned by shuffles.
+__device__ void phases_wave(int n, const z2* beta, z2* phase, double* eabs) {
+    const int lane = threadIdx.x & 63, per = (n + 63) / 64, i0 = lane * per, i1 = min(n, i0 + per);
+    auto unit = [&](int i) {
+        const z2 b = beta[i];
+        const double r = i == 0 ? 0.0 : hypot(b.x, b.y);
+        return r != 0.0 ? z2{b.x / r, b.y / r} : z2{1.0, 0.0};
+    };
+    z2 run = {1.0, 0.0};
+    for (int i = i0; i < i1; ++i) run = zmul(run, unit(i));
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+        const z2 left = {__shfl_up(run.x, o, 64), __shfl_up(run.y, o, 64)};
+        if (lane >= o) run = zmul(left, run);
+    }
+    z2 ph = {__shfl_up(run.x, 1, 64), __shfl_up(run.y, 1, 64)};
+    if (lane == 0) ph = {1.0, 0.0};
+    for (int i = i0; i < i1; ++i) {
+        ph = zmul(ph, unit(i));
+        phase[i] = ph;
+        eabs[i] = i == 0 ? 0.0 : hypot(beta[i].x, beta[i].y);
+    }
+}
+
 // Reflector k: H_k = I - tau v v^H on rows [k+1, n), v_0 = 1, H_k^H x = beta e_0 for
 // x = column k rows [k+1, n).  Its vector is kept in column k rows k+2.. below the implicit 1.
 //
@@ -250,32 +329,21 @@ __global__ void scale_matrix(long nn, double s, z2* __restrict__ A) {
 // over the block; column k+2 (whose reflector step k+2 needs) is finished by wavefront 0 while
 // the others form q.  Per step: one pass and three barriers.
 
-// Column access of the tridiagonalisation.  For the L2-resident matrix, loads and stores go
-// through a buffer resource bounded to the column's live rows: rows past the end read as 0 and
-// their stores are dropped by the hardware, so the row loops need no per-lane branches (with
-// branches the compiler serialises every store behind a full vmcnt wait).  The LDS-resident
-// matrix uses plain accesses with the same guard.
+// Column access of the tridiagonalisation on one workgroup: loads and stores go through a buffer
+// resource bounded to the column's live rows: rows past the end read as 0 and their stores are
+// dropped by the hardware, so the row loops need no per-lane branches (with branches the compiler
+// serialises every store behind a full vmcnt wait).
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-template <bool LM>
 struct ColumnView {
-    z2* base;
-    int len;
     __amdgpu_buffer_rsrc_t rs;
-    __device__ ColumnView(z2* b, int l) : base(b), len(l) {
-        if (!LM) rs = __builtin_amdgcn_make_buffer_rsrc(b, 0, l * 16, 0x00020000);
-    }
+    __device__ ColumnView(z2* b, int l) : rs(__builtin_amdgcn_make_buffer_rsrc(b, 0, l * 16, 0x00020000)) {}
     __device__ z2 load(int i) const {
-        if (LM) return i < len ? base[i] : z2{0.0, 0.0};
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, i * 16, 0, 0);
         z2 r;
         __builtin_memcpy(&r, &v, 16);
         return r;
     }
     __device__ void store(int i, z2 a) const {
-        if (LM) {
-            if (i < len) base[i] = a;
-            return;
-        }
         u32x4 v;
         __builtin_memcpy(&v, &a, 16);
         __builtin_amdgcn_raw_buffer_store_b128(v, rs, i * 16, 0, 0);
@@ -285,12 +353,12 @@ struct ColumnView {
 // Wavefront 0: finish column j (rows [j, n)) with reflector j-1 (vn, q = p - f vn, if tn != 0),
 // record d[j], then form reflector j into vout (and column j's storage) when j <= n-3.
 // Returns tau_j (0 when there is none).  Lane l holds rows j + l + 64 t.
-template <int RPL, bool LM>
+template <int RPL>
 __device__ double column_step(z2* M, int n, int j, double tn, const z2* vn, const z2* p, double f, z2* vout,
                               double* d, z2* beta, double* tau) {
     const int lane = threadIdx.x & 63;
     const int L = n - j;
-    const ColumnView<LM> col(M + j + static_cast<long>(j) * n, L);
+    const ColumnView col(M + j + static_cast<long>(j) * n, L);
     z2 a[RPL];
 #pragma unroll
     for (int t = 0; t < RPL; ++t) a[t] = col.load(lane + 64 * t);
@@ -328,23 +396,16 @@ __device__ double column_step(z2* M, int n, int j, double tn, const z2* vn, cons
     if (tail == 0.0) {
         if (lane == 0) beta[j + 1] = x0;
     } else {
-        const double a0 = hypot(x0.x, x0.y);
-        const double xnorm = sqrt(tail + a0 * a0);
-        const double ia0 = a0 == 0.0 ? 0.0 : div_ulp(1.0, a0);
-        const z2 ph = a0 == 0.0 ? z2{1.0, 0.0} : z2{x0.x * ia0, x0.y * ia0};
-        const z2 b = {-ph.x * xnorm, -ph.y * xnorm};
-        const z2 u0 = {x0.x - b.x, x0.y - b.y};
-        const double iu2 = div_ulp(1.0, u0.x * u0.x + u0.y * u0.y);
-        tj = div_ulp(2.0, 1.0 + tail * iu2);
+        const Reflector h = reflector(x0, tail);
+        tj = h.tau;
 #pragma unroll
         for (int t = 0; t < RPL; ++t) {
             const int i = lane + 64 * t;
-            const z2 w = i == 1 ? z2{1.0, 0.0}
-                                : z2{(a[t].x * u0.x + a[t].y * u0.y) * iu2, (a[t].y * u0.x - a[t].x * u0.y) * iu2};
+            const z2 w = i == 1 ? z2{1.0, 0.0} : zmul(a[t], h.s);
             if (i >= 1 && i < L) vout[i - 1] = w;
             if (i >= 2) col.store(i, w);
         }
-        if (lane == 0) beta[j + 1] = b;
+        if (lane == 0) beta[j + 1] = h.b;
     }
     if (lane == 0) tau[j] = tj;
     return tj;
@@ -357,7 +418,7 @@ __device__ double column_step(z2* M, int n, int j, double tn, const z2* vn, cons
 // store would be a dependent LDS round trip per column); the CB columns' loads are issued
 // together, and their 2 CB wave reductions run side by side with no branch between them.
 // v, q index rows from k+1; vn and p from k+2.
-template <int RPL, int CB, bool LM>
+template <int RPL, int CB>
 __device__ void fused_pass(z2* M, int n, int k, double tk, const z2* v, const z2* q, double tn, const z2* vn,
                            z2* p) {
     const int lane = threadIdx.x & 63;
@@ -380,7 +441,7 @@ __device__ void fused_pass(z2* M, int n, int k, double tk, const z2* v, const z2
 #pragma unroll
         for (int b = 0; b < CB; ++b) {
             const int c = min(c0 + b, len - 1);  // a missing column re-reads the last one (unused)
-            const ColumnView<LM> col(M + static_cast<long>(base + c) * n + base, len);
+            const ColumnView col(M + static_cast<long>(base + c) * n + base, len);
 #pragma unroll
             for (int t = 0; t < RPL; ++t) a[b][t] = col.load(lane + 64 * t);
             qj[b] = tk != 0.0 ? q[c + 1] : z2{0.0, 0.0};
@@ -406,7 +467,7 @@ __device__ void fused_pass(z2* M, int n, int k, double tk, const z2* v, const z2
 #pragma unroll
             for (int b = 0; b < CB; ++b) {
                 if (c0 + b < len) {
-                    const ColumnView<LM> col(M + static_cast<long>(base + c0 + b) * n + base, len);
+                    const ColumnView col(M + static_cast<long>(base + c0 + b) * n + base, len);
 #pragma unroll
                     for (int t = 0; t < RPL; ++t) col.store(lane + 64 * t, a[b][t]);
                 }
@@ -430,7 +491,7 @@ __device__ void fused_pass(z2* M, int n, int k, double tk, const z2* v, const z2
 // A (n x n, ld n, full storage, Hermitian up to rounding) -> d (diagonal), beta (sub-diagonal,
 // beta[i] couples i-1 and i), tau (reflectors, kept in A below the sub-diagonal), the real
 // tridiagonal |beta| in eabs and the phases D in phase (T = D Tr D^H).  RPL >= ceil(n / 64).
-template <bool LM, int RPL>
+template <int RPL>
 __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double* d, z2* beta, double* tau,
                                                            z2* phase, double* eabs) {
     constexpr int CB = RPL <= 2 ? 4 : (RPL <= 4 ? 2 : 1);
@@ -440,17 +501,13 @@ __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double*
     z2* q = sh + 2 * n;
     z2* p = sh + 3 * n;
     double& tnext = *reinterpret_cast<double*>(sh + 4 * n + 16);  // sh + 4n .. 4n + 15: spare
-    z2* M = LM ? sh + 4 * n + 17 : A;
+    z2* M = A;
     // d, beta and tau are kept in LDS and written to global memory once at the end
-    z2* sbeta = sh + 4 * n + 17 + (LM ? static_cast<long>(n) * n : 0);
+    z2* sbeta = sh + 4 * n + 17;
     double* sd = reinterpret_cast<double*>(sbeta + n);
     double* stau = sd + n;
     const int tid = threadIdx.x, nt = blockDim.x, wv = tid >> 6;
     const long nn = static_cast<long>(n) * n;
-    if (LM) {
-        for (long e = tid; e < nn; e += nt) M[e] = A[e];
-        __syncthreads();
-    }
     // Hermitian part: (A + A^H) / 2, real diagonal
     for (long e = tid; e < nn; e += nt) {
         const int i = static_cast<int>(e % n), j = static_cast<int>(e / n);
@@ -480,7 +537,7 @@ __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double*
     } else {
         // reflector 0 (column 0 needs no update)
         if (wv == 0) {
-            const double t0 = column_step<RPL, LM>(M, n, 0, 0.0, nullptr, nullptr, 0.0, vb0, sd, sbeta, stau);
+            const double t0 = column_step<RPL>(M, n, 0, 0.0, nullptr, nullptr, 0.0, vb0, sd, sbeta, stau);
             if ((tid & 63) == 0) tnext = t0;
         }
         __syncthreads();
@@ -493,9 +550,9 @@ __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double*
             const bool one_row = RPL > 1 && n - k - 2 <= 64;
             if (tk != 0.0 || tn != 0.0) {
                 if (one_row)
-                    fused_pass<1, 4, LM>(M, n, k, tk, v, q, tn, vn, p);
+                    fused_pass<1, 4>(M, n, k, tk, v, q, tn, vn, p);
                 else
-                    fused_pass<RPL, CB, LM>(M, n, k, tk, v, q, tn, vn, p);
+                    fused_pass<RPL, CB>(M, n, k, tk, v, q, tn, vn, p);
             }
             __syncthreads();
             const int len = n - k - 2;
@@ -508,8 +565,8 @@ __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double*
                     f = 0.5 * tn * wave_sum(part);
                     for (int i = lane; i < len; i += 64) q[i] = {p[i].x - f * vn[i].x, p[i].y - f * vn[i].y};
                 }
-                const double tj = one_row ? column_step<1, LM>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau)
-                                          : column_step<RPL, LM>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau);
+                const double tj = one_row ? column_step<1>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau)
+                                          : column_step<RPL>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau);
                 if (lane == 0) tnext = tj;
             }
             __syncthreads();
@@ -526,24 +583,400 @@ __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double*
         beta[i] = sbeta[i];
         tau[i] = stau[i];
     }
-    if (tid == 0) {
-        z2 ph = {1.0, 0.0};
-        phase[0] = ph;
-        eabs[0] = 0.0;
-        for (int i = 1; i < n; ++i) {
-            const z2 b = sbeta[i];
-            const double r = hypot(b.x, b.y);
-            eabs[i] = r;
-            if (r != 0.0) ph = zmul(ph, z2{b.x / r, b.y / r});
-            phase[i] = ph;
-        }
-    }
-    if (LM)
-        for (long e = tid; e < nn; e += nt) A[e] = M[e];
+    if (wv == 0) phases_wave(n, sbeta, phase, eabs);
 }
 
-// ---------------------------------------------------------------- 3b. tridiagonalisation over several CUs ----
-// The same reduction with the matrix spread over the LDS of W workgroups: column j lives in
+// ---------------------------------------------------------------- 3b. tridiagonalisation in registers ----
+// The same reduction with every column of the matrix in the registers of one wavefront for the whole
+// reduction (RPL >= ceil(n / 64) rows a lane), on one workgroup (tridiag_cu) or spread
+// over several CUs (tridiag_grid).  Per step the wavefronts apply the rank-2 update to their columns
+// and form their entries of p; the owner of the next pivot column also hands that out; wavefront 0
+// then forms q and the next reflector.  A reflector that is the identity (tau = 0) is kept as a zero
+// vector, so the steps have no cases.
+
+// Wavefront 0, p (the sum of NP parts `stride` apart) and the pivot column pc (entries of rows base..)
+// gathered in LDS: p scaled by tn, f = tn vn^H p / 2, q = p - f vn, the pivot column with reflector
+// k + 1, then reflector `base` into vout.  Row set t covers entries lane + 64 t < len.  Returns tau; d,
+// the next beta and tau go to `out` if this workgroup is the writer.
+struct StepOut {
+    double* d;
+    z2* beta;  // LDS
+    double* tau;
+};
+template <int RPL, int NP>
+__device__ double reflector_step(int base, int len, int n, double tn, const z2* p, int stride, const z2* pc, const z2* vn, z2* q,
+                                 z2* vout, const StepOut& out, bool writer) {
+    const int lane = threadIdx.x & 63;
+    z2 pr[RPL], w[RPL], c[RPL];
+#pragma unroll
+    for (int t = 0; t < RPL; ++t) {
+        pr[t] = w[t] = c[t] = {0.0, 0.0};
+        if (64 * t < len) {
+            const int i = min(lane + 64 * t, len - 1);
+            z2 x[NP];
+#pragma unroll
+            for (int u = 0; u < NP; ++u) x[u] = p[u * stride + i];
+            w[t] = vn[i];
+            c[t] = pc[i];
+#pragma unroll
+            for (int u = 0; u < NP; ++u) {
+                pr[t].x += x[u].x;
+                pr[t].y += x[u].y;
+            }
+            pr[t] = {tn * pr[t].x, tn * pr[t].y};
+        }
+    }
+    double part = 0.0;
+#pragma unroll
+    for (int t = 0; t < RPL; ++t)
+        if (lane + 64 * t < len) part += w[t].x * pr[t].x + w[t].y * pr[t].y;
+    const double f = 0.5 * tn * wave_sum(part);
+#pragma unroll
+    for (int t = 0; t < RPL; ++t) pr[t] = {pr[t].x - f * w[t].x, pr[t].y - f * w[t].y};
+    const z2 q0 = {read_lane(pr[0].x, 0), read_lane(pr[0].y, 0)};
+    double tail = 0.0;
+#pragma unroll
+    for (int t = 0; t < RPL; ++t) {  // the leading entry of a reflector is 1 (p = 0 for a zero one)
+        const int i = lane + 64 * t;
+        const z2 t1 = zmulc(w[t], q0);
+        c[t].x -= t1.x + pr[t].x;
+        c[t].y -= t1.y + pr[t].y;
+        if (i < len) q[i] = pr[t];
+        if (i >= 2 && i < len) tail += c[t].x * c[t].x + c[t].y * c[t].y;
+    }
+    const z2 x0 = {read_lane(c[0].x, 1), read_lane(c[0].y, 1)};
+    if (writer && lane == 0) out.d[base] = c[0].x;
+    if (base >= n - 2) {
+        if (base == n - 2 && writer && lane == 0) out.beta[n - 1] = x0;
+        return 0.0;
+    }
+    tail = wave_sum(tail);
+    Reflector h{x0, {0.0, 0.0}, 0.0};
+    if (tail != 0.0) h = reflector(x0, tail);
+#pragma unroll
+    for (int t = 0; t < RPL; ++t) {
+        const int i = lane + 64 * t;
+        z2 w1 = zmul(c[t], h.s);
+        if (t == 0 && i == 1) w1 = {tail != 0.0 ? 1.0 : 0.0, 0.0};
+        if (i >= 1 && i < len) vout[i - 1] = w1;
+    }
+    if (writer && lane == 0) {
+        out.beta[base + 1] = h.b;
+        out.tau[base] = h.tau;
+    }
+    return h.tau;
+}
+
+// Entry (r, c) of (A + A^H) / 2, real on the diagonal.
+__device__ __forceinline__ z2 herm_entry(const z2* A, int n, int r, int c) {
+    const z2 a = A[r + static_cast<long>(c) * n], b = A[c + static_cast<long>(r) * n];
+    return r == c ? z2{a.x, 0.0} : z2{0.5 * (a.x + b.x), 0.5 * (a.y - b.y)};
+}
+
+// The first reflector, of column 0, by wavefront 0 as a step of zero p and reflector.
+template <int RPL>
+__device__ double first_reflector(const z2* A, int n, z2* p, z2* pc, z2* v, z2* q, z2* vout, const StepOut& out,
+                                  bool writer) {
+    const int lane = threadIdx.x & 63;
+    for (int i = lane; i < n; i += 64) {
+        p[i] = v[i] = q[i] = {0.0, 0.0};
+        pc[i] = herm_entry(A, n, i, 0);
+    }
+    wave_fence();
+    const double t0 = reflector_step<RPL, 1>(0, n, n, 0.0, p, 0, pc, v, q, vout, out, writer);
+    if (writer && lane == 0) {
+        out.beta[0] = {0.0, 0.0};
+        out.tau[n - 2] = 0.0;
+        out.tau[n - 1] = 0.0;
+    }
+    return t0;
+}
+
+// One workgroup of 8 wavefronts, n <= 128: column w + 8 (CPW - 1 - c) is the c-th of wavefront w and
+// row n - 1 - lane - 64 t the t-th of a lane, so that what is left of the trailing block are the first
+// columns of every wavefront and the first row sets.  B is Hermitian, so p = B v is summed over the
+// columns a wavefront owns, lane by lane, and over the wavefronts by wavefront 0: no sum across lanes.
+// Against a kernel of 16 wavefronts that kept the matrix in LDS and summed each p_c across lanes:
+// n = 96 (a 48-band solve) 351 -> 219 us, n = 64 166 -> 95, n = 16 34 -> 23; bound by the issue of the
+// FP64 updates on one CU (about 70 us at n = 96) and by the serial chain of reflector_step.
+constexpr int kCuWaves = 8, kCuMax = 128;
+
+template <int CPW, int RPL>
+__global__ __launch_bounds__(64 * kCuWaves) void tridiag_cu(const z2* __restrict__ A, int n, z2* R, double* d, z2* beta,
+                                                            double* tau, z2* phase, double* eabs) {
+    __shared__ z2 vb[2][kCuMax + 1], q[kCuMax + 1], p[kCuWaves * kCuMax], pc[kCuMax], sbeta[kCuMax];
+    __shared__ double stau;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    z2 a[CPW][RPL];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+#pragma unroll
+        for (int t = 0; t < RPL; ++t) {
+            const int j = wv + kCuWaves * (CPW - 1 - c), r = n - 1 - lane - 64 * t;
+            a[c][t] = j < n && r >= 0 ? herm_entry(A, n, r, j) : z2{0.0, 0.0};
+        }
+    const StepOut out{d, sbeta, tau};
+    if (wv == 0) {
+        const double t0 = first_reflector<RPL>(A, n, p, pc, vb[1], q, vb[0], out, true);
+        if (lane == 0) stau = t0;
+    }
+    __syncthreads();
+    double tn = stau;
+    z2* v = vb[1];   // reflector k
+    z2* vn = vb[0];  // reflector k + 1
+    for (int k = -1; k <= n - 3; ++k) {
+        const int len = n - k - 2, base = k + 2;
+        z2 vi[RPL], qi[RPL];
+#pragma unroll
+        for (int t = 0; t < RPL; ++t) {  // dead rows: zeros, so that they stay as they are
+            vi[t] = qi[t] = {0.0, 0.0};
+            if (64 * t < len) {
+                const int i = len - 1 - lane - 64 * t;
+                const int ic = max(i, 0);
+                vi[t] = v[ic + 1];
+                qi[t] = q[ic + 1];
+                if (i < 0) vi[t] = qi[t] = {0.0, 0.0};
+            }
+        }
+        z2 s[RPL];
+#pragma unroll
+        for (int t = 0; t < RPL; ++t) s[t] = {0.0, 0.0};
+#pragma unroll
+        for (int c = 0; c < CPW; ++c) {
+            const int j = wv + kCuWaves * (CPW - 1 - c);
+            if (j < base || j >= n) continue;
+            const z2 qj = q[j - base + 1], vj = v[j - base + 1], wj = vn[j - base];
+#pragma unroll
+            for (int t = 0; t < RPL; ++t) {
+                if (64 * t >= len) break;
+                const z2 t1 = zmulc(vi[t], qj), t2 = zmulc(qi[t], vj);
+                a[c][t].x -= t1.x + t2.x;
+                a[c][t].y -= t1.y + t2.y;
+                s[t].x += a[c][t].x * wj.x - a[c][t].y * wj.y;
+                s[t].y += a[c][t].x * wj.y + a[c][t].y * wj.x;
+            }
+            if (j == base) {
+#pragma unroll
+                for (int t = 0; t < RPL; ++t) {
+                    const int i = len - 1 - lane - 64 * t;
+                    if (i >= 0) pc[i] = a[c][t];
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < RPL; ++t) {
+            const int i = len - 1 - lane - 64 * t;
+            if (i >= 0) p[wv * kCuMax + i] = s[t];
+        }
+        if (tid >= 64 && tid < 192 && tn != 0.0) {  // reflector k + 1, below its leading 1
+            const int i = tid - 63;
+            if (i < len) R[base + i + static_cast<long>(base - 1) * n] = vn[i];
+        }
+        __syncthreads();
+        if (wv == 0) {
+            const double tj = reflector_step<RPL, kCuWaves>(base, len, n, tn, p, kCuMax, pc, vn, q, v, out, true);
+            if (lane == 0) stau = tj;
+        }
+        __syncthreads();
+        tn = stau;
+        z2* t = v;
+        v = vn;
+        vn = t;
+    }
+    if (wv == 0) {
+        for (int i = lane; i < n; i += 64) beta[i] = sbeta[i];
+        phases_wave(n, sbeta, phase, eabs);
+    }
+}
+
+// Several CUs: wavefront w of workgroup g owns columns 2 (8 g + w) and the next (rows lane + 64 t).  A step's p
+// and pivot column are published to all workgroups, and wavefront 0 of each forms q and the next
+// reflector -- the same operations in the same order, so all hold identical values and nothing else
+// has to be broadcast.
+//
+// The exchange needs no barrier and no fence: every 8-byte word that is published carries 32 bits of
+// a double and the step number, is stored and loaded as one relaxed agent-scope atomic, and a reader
+// repeats its loads until every word has the step it waits for.  (A release and an acquire around
+// flags cost two flights and an invalidation of the caches a step; loads of workgroup scope by
+// workgroups that share an XCD's L2 hit stale lines of the CU's own cache.)  Words are double-buffered
+// by step parity: a workgroup publishes step s + 2 only after every other one that takes part in
+// s + 1 has published s + 1, i.e. has gathered s.  The words are zeroed before the launch; steps
+// count from 1.
+//
+// A workgroup whose columns are all reduced ends; the last one, which ends last, writes the outputs
+// (d, beta, tau, phases, and the reflectors into R, n x n, column k rows k+2..).  At most one
+// workgroup per CU, so all are resident on an otherwise idle device; the wait is bounded (about a
+// second) and sets *fail instead of waiting forever, after which nobody waits any more, so the kernel
+// always drains; the host then redoes the solve on one workgroup.
+// Against a kernel with the matrix in LDS and a grid barrier per step: n = 320 1.86 -> 1.42 ms, n = 160
+// 0.74 -> 0.53 ms; a step at n = 320 is 10,500 cycles, of which the flight of the words through memory
+// takes half, the update a quarter and reflector_step a fifth.  Workgroups of 32 columns took 1.60 ms,
+// of 8 columns (twice as many) 1.39 ms.
+constexpr int kGridWaves = 8, kGridCols = 16;  // wavefronts and columns per workgroup
+constexpr int kGridMax = 512;                  // larger matrices do not fit the registers of its workgroups
+
+typedef unsigned long long u64;
+
+__device__ __forceinline__ void publish(u64* w, u64 tag, int part) {
+    __hip_atomic_store(w, tag | static_cast<unsigned>(part), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 peek(const u64* w) {
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// One more failed poll: whether to give up (somebody has, or the wait is over).
+__device__ __forceinline__ bool give_up(unsigned spins, int* fail) {
+    const int f =
+        __builtin_amdgcn_readfirstlane(__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (f == 0 && spins <= (1u << 20)) return false;
+    if ((threadIdx.x & 63) == 0) atomicExch(fail, 1);
+    return true;
+}
+
+template <int RPL>
+__global__ __launch_bounds__(64 * kGridWaves) void tridiag_grid(const z2* __restrict__ A, int n, z2* R, double* d,
+                                                                z2* beta, double* tau, z2* phase, double* eabs,
+                                                                u64* xP, u64* xC, int* fail) {  // 2 x 4 n words each
+    constexpr int CPW = kGridCols / kGridWaves, cols = kGridCols;
+    extern __shared__ z2 sh[];
+    z2* v = sh;                                             // reflector k
+    z2* vn = sh + (n + 1);                                  // reflector k + 1
+    z2* q = sh + 2 * (n + 1);
+    z2* p = sh + 3 * (n + 1);
+    z2* pc = p + n;
+    z2* sbeta = pc + n;                                     // the writer's
+    double& stau = *reinterpret_cast<double*>(sbeta + n);   // tau of the next reflector
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j0 = blockIdx.x * cols + CPW * wv;            // this wavefront's first column
+    const int last = blockIdx.x * cols + cols - 1;
+    const bool writer = blockIdx.x == gridDim.x - 1;
+    z2 a[CPW][RPL];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+#pragma unroll
+        for (int t = 0; t < RPL; ++t) {
+            const int r = lane + 64 * t;
+            a[c][t] = j0 + c < n && r < n ? herm_entry(A, n, r, j0 + c) : z2{0.0, 0.0};
+        }
+    const StepOut out{d, sbeta, tau};
+    if (wv == 0) {
+        const double t0 = first_reflector<RPL>(A, n, p, pc, v, q, vn, out, writer);
+        if (lane == 0) stau = t0;
+    }
+    __syncthreads();
+    double tn = stau;
+    bool waiting = true;
+    for (int k = -1; k <= n - 3; ++k) {
+        const int len = n - k - 2, base = k + 2;
+        const u64 tag = static_cast<u64>(k + 2) << 32;
+        u64* P = xP + static_cast<long>(k & 1) * 4 * n;
+        u64* Cc = xC + static_cast<long>(k & 1) * 4 * n;
+        if (j0 + CPW > base && j0 < n) {
+            // columns already reduced, or past the end, are carried along and not published
+            z2 qj[CPW], vj[CPW];
+#pragma unroll
+            for (int c = 0; c < CPW; ++c) {
+                const int i = min(max(j0 + c - base, 0), len - 1) + 1;
+                qj[c] = q[i];
+                vj[c] = v[i];
+            }
+            z2 vi[RPL], qi[RPL], w[RPL];
+#pragma unroll
+            for (int t = 0; t < RPL; ++t) {
+                vi[t] = qi[t] = w[t] = {0.0, 0.0};
+                if (64 * t + 63 >= base && 64 * t < n) {
+                    const int ic = min(max(lane + 64 * t - base, 0), len - 1);
+                    vi[t] = v[ic + 1];
+                    qi[t] = q[ic + 1];
+                    w[t] = vn[ic];
+                }
+            }
+            double s[2 * CPW];
+#pragma unroll
+            for (int u = 0; u < 2 * CPW; ++u) s[u] = 0.0;
+#pragma unroll
+            for (int t = 0; t < RPL; ++t) {
+                const int i = lane + 64 * t - base;
+                if (i >= 0 && i < len) {
+#pragma unroll
+                    for (int c = 0; c < CPW; ++c) {
+                        const z2 t1 = zmulc(vi[t], qj[c]), t2 = zmulc(qi[t], vj[c]);
+                        a[c][t].x -= t1.x + t2.x;
+                        a[c][t].y -= t1.y + t2.y;
+                        s[2 * c] += a[c][t].x * w[t].x + a[c][t].y * w[t].y;
+                        s[2 * c + 1] += a[c][t].x * w[t].y - a[c][t].y * w[t].x;
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < CPW; ++c) {
+                if (j0 + c != base) continue;
+#pragma unroll
+                for (int t = 0; t < RPL; ++t) {
+                    const int i = lane + 64 * t - base;
+                    if (i >= 0 && i < len) {
+                        publish(Cc + i, tag, __double2loint(a[c][t].x));
+                        publish(Cc + n + i, tag, __double2hiint(a[c][t].x));
+                        publish(Cc + 2 * n + i, tag, __double2loint(a[c][t].y));
+                        publish(Cc + 3 * n + i, tag, __double2hiint(a[c][t].y));
+                    }
+                }
+            }
+            // lane span u, u = 2 c + (re, im); its first two lanes publish the halves
+            const double x = wave_multi_sum<2 * CPW>(s, lane);
+            constexpr int span = 64 / (2 * CPW);
+            const int u = lane / span, j = j0 + (u >> 1);
+            if (lane % span < 2 && j >= base && j < n)
+                publish(P + (2 * (u & 1) + (lane & 1)) * n + j - base, tag,
+                        (lane & 1) ? __double2hiint(x) : __double2loint(x));
+        }
+        // No column of this workgroup takes part in the next step: it has published its last words and
+        // must not wait for this step's, which others may overwrite without waiting for it
+        if (!writer && last <= base) return;
+        if (writer && tn != 0.0)  // reflector k + 1, below its leading 1
+            for (int i = tid + 1; i < len; i += 64 * kGridWaves) R[base + i + static_cast<long>(base - 1) * n] = vn[i];
+        {  // wavefront w gathers word w mod 4 of p (w < 4) or of the pivot column
+            const u64* src = (wv < 4 ? P : Cc) + (wv & 3) * n;
+            u64 x[RPL];
+            for (unsigned spins = 0;; ++spins) {
+                bool here = true;
+#pragma unroll
+                for (int t = 0; t < RPL; ++t)  // past the end: the last entry again
+                    x[t] = 64 * t < len ? peek(src + min(lane + 64 * t, len - 1)) : tag;
+#pragma unroll
+                for (int t = 0; t < RPL; ++t) here = here && (x[t] >> 32) == (tag >> 32);
+                if (!waiting || __all(here)) break;
+                if (give_up(spins, fail)) {
+                    waiting = false;
+                    break;
+                }
+            }
+            unsigned* dst = reinterpret_cast<unsigned*>(wv < 4 ? p : pc) + (wv & 3);
+#pragma unroll
+            for (int t = 0; t < RPL; ++t)
+                if (lane + 64 * t < len) dst[4 * (lane + 64 * t)] = static_cast<unsigned>(x[t]);
+        }
+        __syncthreads();
+        if (wv == 0) {
+            const double tj = reflector_step<RPL, 1>(base, len, n, tn, p, 0, pc, vn, q, v, out, writer);
+            if (lane == 0) stau = tj;
+        }
+        __syncthreads();
+        tn = stau;
+        z2* t = v;
+        v = vn;
+        vn = t;
+    }
+    if (writer && wv == 0) {
+        for (int i = lane; i < n; i += 64) beta[i] = sbeta[i];
+        phases_wave(n, sbeta, phase, eabs);
+    }
+}
+
+// ---------------------------------------------------------------- 3c. tridiagonalisation over the LDS of many CUs ----
+// Matrices too large for the registers of one XCD (3b).  The same reduction with the matrix spread
+// over the LDS of W workgroups: column j lives in
 // workgroup j mod W (all rows), so the passes run at LDS speed on W CUs instead of at one CU's
 // L2 bandwidth.  Per step: every workgroup updates its own columns and forms its entries of p;
 // the owner of the next pivot column also publishes that column.  One grid barrier; then every
@@ -784,18 +1217,8 @@ __global__ __launch_bounds__(kThreads) void tridiag_coop(const z2* __restrict__ 
         vn = t;
         __syncthreads();
     }
-    if (writer && tid == 0) {
-        z2 ph = {1.0, 0.0};
-        phase[0] = ph;
-        eabs[0] = 0.0;
-        for (int i = 1; i < n; ++i) {
-            const z2 b = beta[i];
-            const double r = hypot(b.x, b.y);
-            eabs[i] = r;
-            if (r != 0.0) ph = zmul(ph, z2{b.x / r, b.y / r});
-            phase[i] = ph;
-        }
-    }
+    __syncthreads();
+    if (writer && wv == 0) phases_wave(n, beta, phase, eabs);
 }
 
 __global__ void zero_words(unsigned* a, int n) {
@@ -1197,7 +1620,7 @@ Layout layout(int n, int nvec) {
                                 size_t(n) * 8, size_t(n) * 8, size_t(n) * 8, size_t(nvec) * 8,  // d e tau w
                                 nv * 8, nv * 8, nv * 8, nv * 8, nv * 8, nv * 4,  // Zt U1 U2 U3 LO SW
                                 size_t(n) * 16, size_t(n) * 16, 64,               // beta phase err
-                                size_t(n) * 32, size_t(n) * 32, (size_t(n) + 1) * 128};  // exchange p, pivot; give-up word, W <= n flags
+                                size_t(n) * 64, size_t(n) * 64, (size_t(n) + 1) * 128};  // exchange p, pivot; give-up word, W <= n flags or ids
     Layout L{};
     size_t o = 0;
     for (int i = 0; i < B_COUNT; ++i) {
@@ -1208,7 +1631,7 @@ Layout layout(int n, int nvec) {
     return L;
 }
 
-size_t tridiag_lds(int n, bool lm) { return (6 * static_cast<size_t>(n) + 17 + (lm ? static_cast<size_t>(n) * n : 0)) * 16; }
+size_t tridiag_lds(int n) { return (6 * static_cast<size_t>(n) + 17) * 16; }
 
 // multi-workgroup launches still to be started with their give-up flag set (test hook), and
 // redos on one workgroup since the process started
@@ -1331,26 +1754,52 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
         double *d = D(B_D), *e = D(B_E), *tau = D(B_TAU), *w = D(B_W);
         z2 *beta = P(B_BETA), *ph = P(B_PH);
         const int rows_lane = (n + 63) / 64;
-        const bool lm = rows_lane <= 2 && tridiag_lds(n, true) <= max_lds;
-        const size_t tl = tridiag_lds(n, lm);
+        const size_t tl = tridiag_lds(n);
         if (tl > max_lds || rows_lane > 16) {
             *err = hipErrorInvalidValue;
             return -1;
         }
-        static std::atomic<bool> lds_raised{false};  // set once per process; the attribute call is idempotent
-        if (!lds_raised && max_lds > 65536) {
-            if (!ok(hipFuncSetAttribute(reinterpret_cast<const void*>(&tridiag_kernel<true, 1>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds))) ||
-                !ok(hipFuncSetAttribute(reinterpret_cast<const void*>(&tridiag_kernel<true, 2>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds))))
-                return -1;
-            lds_raised = true;
-        }
-            // several CUs when the matrix does not fit one CU's LDS: column j on workgroup j mod W,
-        // about 16 columns (one per wavefront) each, fewer when LDS is short
+        // one CU's registers, those of several CUs, the LDS of many CUs; or (n <= 2, and a solve redone
+        // after a wait that gave up) one workgroup on the matrix in L2
         z2* refl = C;  // where the reflectors end up
-        bool coop_done = false;
-        if (!lm && n >= 100 && multi_wg_ok) {
+        bool grid_done = false;
+        if (n >= 3 && n <= kCuMax) {
+            refl = T1;
+#define Q3X_TRC(CP, RP) \
+    hipLaunchKernelGGL((tridiag_cu<CP, RP>), dim3(1), dim3(64 * kCuWaves), 0, st, C, n, T1, d, beta, tau, ph, e)
+            if (n <= 16) Q3X_TRC(2, 1);
+            else if (n <= 32) Q3X_TRC(4, 1);
+            else if (n <= 64) Q3X_TRC(8, 1);
+            else if (n <= 96) Q3X_TRC(12, 2);
+            else Q3X_TRC(16, 2);
+#undef Q3X_TRC
+        } else if (n > kCuMax && n <= kGridMax && multi_wg_ok && n / kGridCols < num_cus_hint) {
+            // word 1: the give-up flag; the words of p and of the pivot column lie before it
+            unsigned* bar = reinterpret_cast<unsigned*>(base + L.off[B_BAR]);
+            u64 *xp = reinterpret_cast<u64*>(base + L.off[B_XP]), *xc = reinterpret_cast<u64*>(base + L.off[B_XC]);
+            int* fail = reinterpret_cast<int*>(bar + 1);
+            const int words = static_cast<int>((L.off[B_BAR] - L.off[B_XP]) / 4) + 2;
+            hipLaunchKernelGGL(zero_words, dim3((words + 255) / 256), dim3(256), 0, st, reinterpret_cast<unsigned*>(xp),
+                               words);
+            if (!ok(hipGetLastError())) return -1;
+            if (take_forced_giveup()) {
+                hipLaunchKernelGGL(set_word, dim3(1), dim3(64), 0, st, fail, 1);
+                if (!ok(hipGetLastError())) return -1;
+            }
+            const size_t lds = (6 * static_cast<size_t>(n) + 4) * 16;
+#define Q3X_TRG(RP)                                                                                            \
+    hipLaunchKernelGGL(tridiag_grid<RP>, dim3((n + kGridCols - 1) / kGridCols), dim3(64 * kGridWaves), lds, st, C, n,   \
+                       T1, d, beta, tau, ph, e, xp, xc, fail)
+            if (rows_lane <= 3) Q3X_TRG(3);
+            else if (rows_lane <= 4) Q3X_TRG(4);
+            else if (rows_lane <= 5) Q3X_TRG(5);
+            else if (rows_lane <= 6) Q3X_TRG(6);
+            else Q3X_TRG(8);
+#undef Q3X_TRG
+            if (!ok(hipGetLastError())) return -1;
+            grid_done = true;
+            refl = T1;
+        } else if (n > kGridMax && multi_wg_ok) {
             const long room = static_cast<long>(max_lds / 16) - 5L * n - 16;
             const int ncl = static_cast<int>(std::min<long>(16, room / n));
             if (ncl >= 1) {
@@ -1381,24 +1830,21 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
                     hipLaunchKernelGGL(tridiag_coop, dim3(W), dim3(kThreads), lds, st, Cc, n, R, d, beta, tau, ph, e,
                                        xp, xc, bar, fail);
                     if (!ok(hipGetLastError())) return -1;
-                    coop_done = true;
+                    grid_done = true;
                     refl = T1;
                 }
             }
         }
-#define Q3X_TRD(LMV, R) \
-        hipLaunchKernelGGL((tridiag_kernel<LMV, R>), dim3(1), dim3(kThreads), tl, st, C, n, d, beta, tau, ph, e)
-        if (coop_done) {
-        } else if (lm) {
-            if (rows_lane <= 1) Q3X_TRD(true, 1);
-            else Q3X_TRD(true, 2);
-        } else if (rows_lane <= 1) Q3X_TRD(false, 1);
-        else if (rows_lane <= 2) Q3X_TRD(false, 2);
-        else if (rows_lane <= 4) Q3X_TRD(false, 4);
-        else if (rows_lane <= 6) Q3X_TRD(false, 6);
-        else if (rows_lane <= 8) Q3X_TRD(false, 8);
-        else if (rows_lane <= 12) Q3X_TRD(false, 12);
-        else Q3X_TRD(false, 16);
+#define Q3X_TRD(R) \
+        hipLaunchKernelGGL((tridiag_kernel<R>), dim3(1), dim3(kThreads), tl, st, C, n, d, beta, tau, ph, e)
+        if (refl == T1) {
+        } else if (rows_lane <= 1) Q3X_TRD(1);
+        else if (rows_lane <= 2) Q3X_TRD(2);
+        else if (rows_lane <= 4) Q3X_TRD(4);
+        else if (rows_lane <= 6) Q3X_TRD(6);
+        else if (rows_lane <= 8) Q3X_TRD(8);
+        else if (rows_lane <= 12) Q3X_TRD(12);
+        else Q3X_TRD(16);
     #undef Q3X_TRD
         if (!ok(hipGetLastError())) return -1;
         stage_done(K_EIG_TRIDIAG);
@@ -1433,7 +1879,7 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
         if (!ok(hipGetLastError())) return -1;
         if (!gemm(0, n, nvec, nvec, Yb, n, G, nvec, Y2, n) || !gemm(0, n, nvec, n, Zl, n, Y2, n, X, ldx)) return -1;
         stage_done(K_EIG_BACK);
-        int coop_fail = 0;
+        int grid_fail = 0;
         const size_t wb = static_cast<size_t>(nvec) * 8;
         char* sw = pin ? pin->take(wb + 16, st) : nullptr;
         if (pin && !sw) {
@@ -1442,19 +1888,19 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
         }
         double* w_dst = sw ? reinterpret_cast<double*>(sw) : w_host;
         double* sdev_dst = sw ? reinterpret_cast<double*>(sw + wb) : sdev_out;
-        int* fail_dst = sw ? reinterpret_cast<int*>(sw + wb + 8) : &coop_fail;
+        int* fail_dst = sw ? reinterpret_cast<int*>(sw + wb + 8) : &grid_fail;
         if (!ok(hipMemcpyAsync(w_dst, w, wb, hipMemcpyDeviceToHost, st)) ||
             !ok(hipMemcpyAsync(sdev_dst, errd, 8, hipMemcpyDeviceToHost, st)) ||
-            (coop_done && !ok(hipMemcpyAsync(fail_dst, base + L.off[B_BAR] + 4, 4, hipMemcpyDeviceToHost, st))) ||
+            (grid_done && !ok(hipMemcpyAsync(fail_dst, base + L.off[B_BAR] + 4, 4, hipMemcpyDeviceToHost, st))) ||
             !ok(hipStreamSynchronize(st)))
             return -1;
         if (sw) {
             std::memcpy(w_host, sw, wb);
             std::memcpy(sdev_out, sw + wb, 8);
-            if (coop_done) std::memcpy(&coop_fail, sw + wb + 8, 4);
+            if (grid_done) std::memcpy(&grid_fail, sw + wb + 8, 4);
             pin->rewind();
         }
-        if (coop_fail) return -2;  // a grid barrier gave up waiting
+        if (grid_fail) return -2;  // a workgroup gave up waiting
         return 0;
     };
     double sdev = 0.0, sdev2 = 0.0;
