@@ -222,6 +222,7 @@ HLocalArgs make_args(const q3x_hamiltonian_s* h, bool fp32) {
     a.stick_i2 = h->stick_i2.as<int>();
     a.stick_col = h->stick_col.as<int>();
     a.col_i1 = h->col_i1.as<int>();
+    a.col_stick = h->col_stick.as<int>();
     a.ent_pw = h->ent_pw.as<int>();
     a.ent_pos = h->ent_pos.as<int>();
     a.ekin = h->ekin.as<double>();
@@ -465,7 +466,7 @@ double device_bytes_held(const q3x_context_s* c, const q3x_hamiltonian_s* h) {
             b += static_cast<double>(d->size());
     }
     if (h) {
-        for (const DevBuf* d : {&h->v64, &h->v32, &h->stick_off, &h->stick_i2, &h->stick_col, &h->col_i1, &h->ent_pw,
+        for (const DevBuf* d : {&h->v64, &h->v32, &h->stick_off, &h->stick_i2, &h->stick_col, &h->col_i1, &h->col_stick, &h->ent_pw,
                                 &h->ent_pos, &h->ekin, &h->outside, &h->beta64, &h->beta32, &h->dblocks, &h->pstart,
                                 &h->psize, &h->poff, &h->zbuf, &h->P, &h->W, &h->gemm_work, &h->io_psi, &h->io_hpsi,
                                 &h->plane_slots, &h->gpack, &h->gout, &h->kb_g, &h->kb_tables, &h->kb_form,
@@ -872,6 +873,10 @@ q3x_status q3x_hamiltonian_prepare_kpoint(q3x_hamiltonian h, q3x_kpoint k) {
         const bool use_tl = !(pk && std::strcmp(pk, "generic") == 0) && plane_tl_supported(n1, n2);
         h->tl64 = use_tl ? plane_tl_config(n1, S.ncol, false, h->ctx->max_lds, h->ctx->num_cus) : PlaneTlConfig{};
         h->tl32 = use_tl ? plane_tl_config(n1, S.ncol, true, h->ctx->max_lds, h->ctx->num_cus) : PlaneTlConfig{};
+        // the planes' pruned form where the occupied sticks and columns allow it and the plane is in LDS
+        const std::vector<int> quarters = use_tl ? plane_tl_quarters(n1, S) : std::vector<int>();
+        h->tl64.quarters = h->tl64.ok && !h->tl64.plane_global && !quarters.empty();
+        h->tl32.quarters = h->tl32.ok && !h->tl32.plane_global && !quarters.empty();
         const bool use_tz = !(pk && std::strcmp(pk, "generic") == 0) && stick_tl_supported(n3);
         h->tz64 = use_tz ? stick_tl_config(n3, false) : StickTlConfig{};
         h->tz32 = use_tz ? stick_tl_config(n3, true) : StickTlConfig{};
@@ -896,6 +901,7 @@ q3x_status q3x_hamiltonian_prepare_kpoint(q3x_hamiltonian h, q3x_kpoint k) {
                   h->stick_i2.upload(S.stick_i2.data(), S.stick_i2.size() * sizeof(int), st, &h->ctx->pin) &&
                   h->stick_col.upload(S.stick_col.data(), S.stick_col.size() * sizeof(int), st, &h->ctx->pin) &&
                   h->col_i1.upload(S.col_i1.data(), S.col_i1.size() * sizeof(int), st, &h->ctx->pin) &&
+                  h->col_stick.upload(quarters.data(), quarters.size() * sizeof(int), st, &h->ctx->pin) &&
                   h->ent_pw.upload(S.ent_pw.data(), S.ent_pw.size() * sizeof(int), st, &h->ctx->pin) &&
                   h->ent_pos.upload(S.ent_pos.data(), S.ent_pos.size() * sizeof(int), st, &h->ctx->pin) &&
                   h->ekin.upload(tkin.data(), tkin.size() * sizeof(double), st, &h->ctx->pin) &&

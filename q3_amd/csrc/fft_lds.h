@@ -143,9 +143,18 @@ struct DftComposite {
         for (int r1 = 1; r1 < A; ++r1)
 #pragma unroll
             for (int k1 = 1; k1 < B; ++k1) {
+                // quarter turns cost no multiplication (the table's cos pi/2 would)
                 const int p = (r1 * k1) % R;
-                const cx<T> w = {T(TwR<R>::c[p]), sgn * T(TwR<R>::s[p])};
-                y[r1][k1] = cmul(y[r1][k1], w);
+                if (4 * p == R) {
+                    y[r1][k1] = cmuli(y[r1][k1], sgn);
+                } else if (2 * p == R) {
+                    y[r1][k1] = {-y[r1][k1].x, -y[r1][k1].y};
+                } else if (4 * p == 3 * R) {
+                    y[r1][k1] = cmuli(y[r1][k1], -sgn);
+                } else {
+                    const cx<T> w = {T(TwR<R>::c[p]), sgn * T(TwR<R>::s[p])};
+                    y[r1][k1] = cmul(y[r1][k1], w);
+                }
             }
 #pragma unroll
         for (int k1 = 0; k1 < B; ++k1) {

@@ -2,7 +2,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "fft_lds.h"
+#include "q3x_internal.h"
 
 namespace q3x {
 
@@ -21,6 +24,7 @@ struct HLocalArgs {
     const int* stick_i2;          // nst
     const int* stick_col;         // nst
     const int* col_i1;            // ncol
+    const int* col_stick;         // stick of (column, quarter element, lane), or -1 (PlaneTlConfig::quarters)
     const int* ent_pw;            // entries (stick order) -> plane-wave index
     const int* ent_pos;           // entries -> stick * n3 + i3
     const double* ekin;           // npw, Ry
@@ -41,7 +45,13 @@ struct PlaneTlConfig {
     size_t lds = 0;
     bool plane_global = false;  // plane too large for LDS: kept in a global slot per workgroup
     size_t plane_bytes = 0;     // bytes of one plane slot
+    // every occupied stick and column lies in the first or the last `quarter` blocks of B of its axis
+    // (plane_tl_quarters): the first stages then run on 2 quarter of their A inputs
+    bool quarters = false;
 };
+// col_stick of a layout whose occupied i1 and i2 lie in the outer quarters of a plane of size n (ncol x
+// 2 quarter x B entries); empty where they do not, or no kernel of that size exists
+std::vector<int> plane_tl_quarters(int n, const StickLayout& s);
 bool plane_tl_supported(int n1, int n2);
 PlaneTlConfig plane_tl_config(int n, int ncol, bool fp32, size_t max_lds, int num_cus);
 // Two-level z-stick kernels (plane_tl.hip) for the n3 the plane sizes list holds.
