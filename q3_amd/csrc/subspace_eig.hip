@@ -1234,23 +1234,37 @@ __global__ void set_word(int* a, int v) {
 }
 
 // ---------------------------------------------------------------- 4. eigenvalues ----
-// Number of eigenvalues of the tridiagonal (d, e2 = e^2) below x (Sturm count of the LDL^T
-// pivots; pivots smaller than pivmin are replaced by -pivmin, as LAPACK's dstebz does).
-__device__ int sturm_count(int n, const double* d, const double* e2, double x, double pivmin) {
-    int c = 0;
-    double q = d[0] - x;
-    if (fabs(q) <= pivmin) q = -pivmin;
-    c += q < 0.0;
-    for (int i = 1; i < n; ++i) {
-        q = (d[i] - x) - div_ulp(e2[i], q);
-        if (fabs(q) <= pivmin) q = -pivmin;
-        c += q < 0.0;
+// Number of eigenvalues below x of the tridiagonal, scaled by a power of two to a norm in [1/2, 1), with
+// de[i] = (d_i, e_i^2): sign changes of p_i = (d_i - x) p_{i-1} - e_i^2 p_{i-2} (Givens).  Each p_i is
+// that of a tridiagonal whose d_i - x and e_i^2 are off by O(eps) relative, like the quotients
+// p_i / p_{i-1} of the LDL^T pivots, but the serial chain is one multiply-add a step instead of a
+// division (133 -> 64 us for the lower half at n = 320, 46 -> 25 us at n = 96).  e_i^2 is kept above
+// 2^-160 (a change of e_i by 2^-80 of the norm), so a zero p_{i-1} is followed by the opposite of
+// p_{i-2}: one change, as it should be.  p and its predecessor are rescaled every eight steps, within
+// which they grow by at most 3^8 and shrink to no less than 2^-810.
+__device__ int sturm_count(int n, const double2* de, double x) {
+    double pp = 1.0, p = de[0].x - x;
+    unsigned c = static_cast<unsigned>(__double2hiint(p)) >> 31;
+    auto step = [&](double2 v) {
+        const double t = fma(v.x - x, p, -v.y * pp);
+        c += static_cast<unsigned>(__double2hiint(t) ^ __double2hiint(p)) >> 31;
+        pp = p;
+        p = t;
+    };
+    int i = 1;
+    for (; i + 8 <= n; i += 8) {
+        double2 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = de[i + u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) step(v[u]);
+        const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(p), fabs(pp)));
+        p = ldexp(p, ex);
+        pp = ldexp(pp, ex);
     }
-    return c;
+    for (; i < n; ++i) step(de[i]);
+    return static_cast<int>(c);
 }
-
-// Gershgorin interval [gl, gu] of the tridiagonal, its norm bound tn and pivmin; lane-parallel
-// over one wavefront, same result in every lane.
 __device__ void tri_bounds(int n, const double* d, const double* e, double& gl, double& gu, double& tn,
                            double& pivmin) {
     const int lane = threadIdx.x & 63;
@@ -1275,23 +1289,23 @@ __device__ void tri_bounds(int n, const double* d, const double* e, double& gl, 
 // wavefront per eigenvalue; each round evaluates 63 interior points of the bracket.
 __global__ __launch_bounds__(64) void bisect_kernel(int n, const double* __restrict__ d, const double* __restrict__ e,
                                                     double* __restrict__ w) {
-    extern __shared__ double tsh[];
-    double* sd = tsh;
-    double* se2 = tsh + n;
+    extern __shared__ double2 tsh[];
     const int lane = threadIdx.x;
-    for (int i = lane; i < n; i += 64) {
-        sd[i] = d[i];
-        se2[i] = i > 0 ? e[i] * e[i] : 0.0;
-    }
-    __syncthreads();
     double gl, gu, tn, pivmin;
     tri_bounds(n, d, e, gl, gu, tn, pivmin);
+    // scaled by 2^-k, exactly
+    const int k = tn > 0.0 ? __builtin_amdgcn_frexp_exp(tn) : 0;
+    for (int i = lane; i < n; i += 64) {
+        const double es = i > 0 ? ldexp(e[i], -k) : 0.0;
+        tsh[i] = {ldexp(d[i], -k), fmax(es * es, 0x1p-160)};
+    }
+    __syncthreads();
     const int target = blockIdx.x + 1;  // lambda_i is the smallest x with count(x) >= i + 1
     double lo = gl, hi = gu;
     for (int round = 0; round < 32; ++round) {
         if (hi - lo <= 2.0 * kEps * fmax(fabs(lo), fabs(hi)) + kEps * tn) break;
         const double x = lane == 63 ? hi : lo + (hi - lo) * static_cast<double>(lane + 1) * (1.0 / 64.0);
-        const int cnt = lane == 63 ? n : sturm_count(n, sd, se2, x, pivmin);
+        const int cnt = lane == 63 ? n : sturm_count(n, tsh, ldexp(x, -k));
         const unsigned long long mask = __ballot(cnt >= target);
         const int f = __ffsll(static_cast<long long>(mask)) - 1;  // lane 63 is always set
         const double nlo = f == 0 ? lo : lo + (hi - lo) * static_cast<double>(f) * (1.0 / 64.0);
@@ -1382,80 +1396,84 @@ __global__ __launch_bounds__(kInvitThreads) void invit_kernel(int n, const doubl
                 // the vector is accurate to about eps |T| / gap.  U1 holds L+, U2 D+, U3 U-.
                 // The divisions are div_ulp's: the recurrences need O(eps) relative error per
                 // operation, and they are the serial chain of this kernel.
-                double dp = d[0] - mu;
-                for (int i = 0; i + 1 < n; ++i) {
-                    if (fabs(dp) < pivmin) dp = dp >= 0.0 ? pivmin : -pivmin;
-                    const double l = div_ulp(e[i + 1], dp);
-                    U1[at(i)] = l;
-                    U2[at(i)] = dp;
-                    dp = (d[i + 1] - mu) - l * e[i + 1];
+                // The two factorisations run side by side, as do the two recurrences for z: each
+                // is a serial chain of divisions, or of loads and products, that leaves the
+                // pipelines idle (n = 320: 210 -> 176 us).  LO holds D-.
+                double dp = d[0] - mu, dm = d[n - 1] - mu;
+                for (int i0 = 0; i0 + 1 < n; i0 += kPf) {
+                    double ef[kPf], df[kPf], eb[kPf], db[kPf];
+#pragma unroll
+                    for (int k = 0; k < kPf; ++k) {
+                        const int i = min(i0 + k, n - 2);
+                        ef[k] = e[i + 1];
+                        df[k] = d[i + 1];
+                        eb[k] = e[n - 1 - i];
+                        db[k] = d[n - 2 - i];
+                    }
+#pragma unroll
+                    for (int k = 0; k < kPf; ++k) {
+                        const int i = i0 + k, ib = n - 1 - i;
+                        if (i + 1 >= n) break;
+                        if (fabs(dp) < pivmin) dp = dp >= 0.0 ? pivmin : -pivmin;
+                        LO[at(ib)] = dm;
+                        if (fabs(dm) < pivmin) dm = dm >= 0.0 ? pivmin : -pivmin;
+                        const double l = div_ulp(ef[k], dp), u = div_ulp(eb[k], dm);
+                        U1[at(i)] = l;
+                        U2[at(i)] = dp;
+                        U3[at(ib)] = u;
+                        dp = (df[k] - mu) - l * ef[k];
+                        dm = (db[k] - mu) - u * eb[k];
+                    }
                 }
                 if (fabs(dp) < pivmin) dp = dp >= 0.0 ? pivmin : -pivmin;
                 U2[at(n - 1)] = dp;
-                double dm = d[n - 1] - mu;
-                double best = fabs(dp + dm - (d[n - 1] - mu));
+                LO[at(0)] = dm;
+                double best = INFINITY;
                 int rt = n - 1;
-                for (int i0 = n - 1; i0 >= 1; i0 -= kPf) {  // steps i = i0, i0-1, ... >= 1
-                    double dpb[kPf];
+                for (int i0 = n - 1; i0 >= 0; i0 -= 2 * kPf) {
+                    double g[2 * kPf], gm[2 * kPf];
 #pragma unroll
-                    for (int k = 0; k < kPf; ++k)
-                        if (i0 - k >= 1) dpb[k] = U2[at(i0 - k - 1)];
+                    for (int k = 0; k < 2 * kPf; ++k) {
+                        const int i = max(i0 - k, 0);
+                        g[k] = U2[at(i)];
+                        gm[k] = LO[at(i)];
+                    }
 #pragma unroll
-                    for (int k = 0; k < kPf; ++k) {
-                        const int i = i0 - k;
-                        if (i < 1) break;
-                        if (fabs(dm) < pivmin) dm = dm >= 0.0 ? pivmin : -pivmin;
-                        const double u = div_ulp(e[i], dm);
-                        U3[at(i)] = u;
-                        dm = (d[i - 1] - mu) - u * e[i];
-                        const double g = fabs(dpb[k] + dm - (d[i - 1] - mu));
-                        if (g < best) {
-                            best = g;
-                            rt = i - 1;
+                    for (int k = 0; k < 2 * kPf; ++k) {
+                        const int i = max(i0 - k, 0);  // entry 0 again is no improvement
+                        const double gamma = fabs(g[k] + gm[k] - (d[i] - mu));
+                        if (gamma < best) {
+                            best = gamma;
+                            rt = i;
                         }
                     }
                 }
-                double z = 1.0, nrm = 1.0;
+                double zd = 1.0, zu = 1.0, nd = 0.0, nu = 0.0;
                 Zt[at(rt)] = 1.0;
-                for (int i0 = rt - 1; i0 >= 0; i0 -= kPf) {
-                    double lb[kPf];
-#pragma unroll
-                    for (int k = 0; k < kPf; ++k)
-                        if (i0 - k >= 0) lb[k] = U1[at(i0 - k)];
+                const int longer = max(rt, n - 1 - rt);
+                for (int s0 = 1; s0 <= longer; s0 += kPf) {  // rows rt - s and rt + s
+                    double lb[kPf], ub[kPf];
 #pragma unroll
                     for (int k = 0; k < kPf; ++k) {
-                        const int i = i0 - k;
-                        if (i < 0) break;
-                        z = -lb[k] * z;
-                        Zt[at(i)] = z;
-                        nrm += z * z;
+                        lb[k] = U1[at(max(rt - s0 - k, 0))];
+                        ub[k] = U3[at(min(rt + s0 + k, n - 1))];
                     }
-                }
-                z = 1.0;
-                for (int i0 = rt + 1; i0 < n; i0 += kPf) {
-                    double ub[kPf];
-#pragma unroll
-                    for (int k = 0; k < kPf; ++k)
-                        if (i0 + k < n) ub[k] = U3[at(i0 + k)];
 #pragma unroll
                     for (int k = 0; k < kPf; ++k) {
-                        const int i = i0 + k;
-                        if (i >= n) break;
-                        z = -ub[k] * z;
-                        Zt[at(i)] = z;
-                        nrm += z * z;
+                        const int a = rt - s0 - k, b = rt + s0 + k;
+                        if (a >= 0) {
+                            zd = -lb[k] * zd;
+                            Zt[at(a)] = zd;
+                            nd += zd * zd;
+                        }
+                        if (b < n) {
+                            zu = -ub[k] * zu;
+                            Zt[at(b)] = zu;
+                            nu += zu * zu;
+                        }
                     }
                 }
-                const double inv = 1.0 / sqrt(nrm);
-                for (int i0 = 0; i0 < n; i0 += kPf) {
-                    double zb[kPf];
-#pragma unroll
-                    for (int k = 0; k < kPf; ++k)
-                        if (i0 + k < n) zb[k] = Zt[at(i0 + k)];
-#pragma unroll
-                    for (int k = 0; k < kPf; ++k)
-                        if (i0 + k < n) Zt[at(i0 + k)] = zb[k] * inv;
-                }
+                U1[at(0)] = 1.0 / sqrt(1.0 + nd + nu);  // the norm, applied by the back-transformation
                 continue;
             }
             // LU with partial pivoting of Tr - mu I: row i keeps (u1 diag, u2, u3 super-diagonals).
@@ -1527,67 +1545,100 @@ __global__ __launch_bounds__(kInvitThreads) void invit_kernel(int n, const doubl
                 const double inv = nrm > 0.0 ? 1.0 / sqrt(nrm) : 0.0;
                 for (int i = 0; i < n; ++i) Zt[at(i)] *= inv;
             }
+            U1[at(0)] = 1.0;
         }
         __syncthreads();
     }
 }
 
 // ---------------------------------------------------------------- 6. back-transformation ----
-// Y[:, c] = H_0 H_1 ... H_{n-3} D Zt[:, c]; one wavefront per column, RPL rows per lane.
+// Y[:, c] = H_0 H_1 ... H_{n-3} D (scale[c] Zt[:, c]); one wavefront per column, RPL rows per lane.
+// Bound by its serial chain: a step is the product's multiply-adds over the rows below the reflector's
+// 1 and one reduction of (re, im) together.  Reflectors are loaded PF at a time, one batch ahead of
+// the batch that is applied (n = 320: 227 -> 140 us, 155 where loads of a masked row are skipped).
 template <int RPL>
 __global__ __launch_bounds__(64) void backtransform_kernel(int n, const z2* __restrict__ A,
                                                            const double* __restrict__ tau,
                                                            const z2* __restrict__ phase,
-                                                           const double* __restrict__ Zt, int nvec,
+                                                           const double* __restrict__ Zt,
+                                                           const double* __restrict__ scale, int nvec,
                                                            z2* __restrict__ Y) {
     const int lane = threadIdx.x, c = blockIdx.x;
+    const double sc = scale[c];
     z2 y[RPL];
 #pragma unroll
     for (int r = 0; r < RPL; ++r) {
         const int i = lane + 64 * r;
         if (i < n) {
-            const double z = Zt[static_cast<long>(i) * nvec + c];
+            const double z = sc * Zt[static_cast<long>(i) * nvec + c];
             const z2 ph = phase[i];
             y[r] = {ph.x * z, ph.y * z};
         } else {
             y[r] = {0.0, 0.0};
         }
     }
-    // reflectors k = n-3 .. 0, PF at a time: their entries are loaded together, then applied in
-    // order, so one L2 round trip serves PF serial steps
-    constexpr int PF = RPL <= 16 ? 32 / RPL : 2;
-    for (int k0 = n - 3; k0 >= 0; k0 -= PF) {
-        z2 vb[PF][RPL];
-        double tb[PF];
+    constexpr int PF = RPL <= 2 ? 8 : RPL < 16 ? 24 / RPL : 1;
+    constexpr int FULL = RPL <= 6 ? RPL - 1 : RPL == 8 ? 6 : RPL - 4;  // blocks of 64 rows surely below n
+    struct Batch {
+        z2 v[PF][RPL];
+        double t[PF];
+    };
+    // Loads are unconditional, so that the wait for one batch leaves the next one in flight: past the
+    // first reflector column 0 again with tau = 0, past the last row that row again.
+    auto load = [&](Batch& b, int k0) {  // reflectors k0 .. k0 - PF + 1
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
-            const int k = k0 - q;
-            tb[q] = k >= 0 ? tau[k] : 0.0;
-            const z2* col = A + static_cast<long>(k >= 0 ? k : 0) * n;
+            const int k = max(k0 - q, 0);
+            const double t = tau[k];
+            b.t[q] = k0 - q >= 0 ? t : 0.0;
+            const z2* col = A + static_cast<long>(k) * n;
 #pragma unroll
-            for (int r = 0; r < RPL; ++r) {
-                const int i = lane + 64 * r;
-                vb[q][r] = (k >= 0 && i > k + 1 && i < n) ? col[i] : z2{i == k + 1 ? 1.0 : 0.0, 0.0};
-            }
+            for (int r = 0; r < RPL; ++r) b.v[q][r] = col[r < FULL ? lane + 64 * r : min(lane + 64 * r, n - 1)];
         }
+    };
+    auto apply = [&](Batch& b, int k0) {
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
-            const double t = tb[q];
-            if (t == 0.0) continue;  // also every k < 0 of the last chunk
-            double sr = 0.0, si = 0.0;
+            const double t = b.t[q];
+            if (t == 0.0) continue;
+            const int one = k0 - q + 1;  // row of the reflector's 1; zeros above it
+            double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int r = 0; r < RPL; ++r) {
-                sr += vb[q][r].x * y[r].x + vb[q][r].y * y[r].y;
-                si += vb[q][r].x * y[r].y - vb[q][r].y * y[r].x;
+                if (64 * r + 63 < one) continue;
+                z2& v = b.v[q][r];
+                if (64 * r <= one || r >= FULL) {
+                    const int i = lane + 64 * r;
+                    v.x = i > one && i < n ? v.x : i == one ? 1.0 : 0.0;
+                    v.y = i > one && i < n ? v.y : 0.0;
+                }
+                s[0] += v.x * y[r].x;
+                s[1] += v.y * y[r].y;
+                s[2] += v.x * y[r].y;
+                s[3] -= v.y * y[r].x;
             }
-            sr = t * wave_sum(sr);
-            si = t * wave_sum(si);
+            double x = swap_sum<true>(s[0] + s[1], s[2] + s[3]);  // lanes 0-31 re, 32-63 im
+            x = swap_sum<false>(x, x);
+            x += dpp_mov<0x140>(x);
+            x += dpp_mov<0x141>(x);
+            x += dpp_mov<0x4E>(x);
+            x += dpp_mov<0xB1>(x);
+            const double sr = t * read_lane(x, 0), si = t * read_lane(x, 32);
 #pragma unroll
             for (int r = 0; r < RPL; ++r) {
-                y[r].x -= vb[q][r].x * sr - vb[q][r].y * si;
-                y[r].y -= vb[q][r].x * si + vb[q][r].y * sr;
+                if (64 * r + 63 < one) continue;
+                y[r].x -= b.v[q][r].x * sr - b.v[q][r].y * si;
+                y[r].y -= b.v[q][r].x * si + b.v[q][r].y * sr;
             }
         }
+    };
+    Batch b0, b1;
+    load(b0, n - 3);
+    for (int k0 = n - 3; k0 >= 0; k0 -= 2 * PF) {
+        load(b1, k0 - PF);
+        apply(b0, k0);
+        load(b0, k0 - 2 * PF);
+        apply(b1, k0 - PF);
     }
 #pragma unroll
     for (int r = 0; r < RPL; ++r) {
@@ -1858,11 +1909,15 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
         z2* Yb = P(B_YB);
         const int rpl = (n + 63) / 64;
     #define Q3X_BT(R)                                                                                              \
-        hipLaunchKernelGGL(backtransform_kernel<R>, dim3(nvec), dim3(64), 0, st, n, refl, tau, ph, D(B_ZT), nvec, Yb)
+        hipLaunchKernelGGL(backtransform_kernel<R>, dim3(nvec), dim3(64), 0, st, n, refl, tau, ph, D(B_ZT), D(B_U1), nvec, Yb)
         if (rpl <= 1) Q3X_BT(1);
         else if (rpl <= 2) Q3X_BT(2);
+        else if (rpl <= 3) Q3X_BT(3);
         else if (rpl <= 4) Q3X_BT(4);
+        else if (rpl <= 5) Q3X_BT(5);
+        else if (rpl <= 6) Q3X_BT(6);
         else if (rpl <= 8) Q3X_BT(8);
+        else if (rpl <= 12) Q3X_BT(12);
         else if (rpl <= 16) Q3X_BT(16);
         else {
             *err = hipErrorInvalidValue;
