@@ -31,7 +31,7 @@ EXTRA = {
     # butterflies with inputs known to be zero: x + 0 folds to x only without signed zeros
     "plane_tl.hip": ["-fno-signed-zeros"],
 }
-SOURCES = ["setup.cpp", "kb_projectors.cpp", "api.cpp", "hlocal.hip", "plane_tl.hip", "zgemm.hip", "zgemm64.hip", "aux_kernels.hip",
+SOURCES = ["setup.cpp", "kb_projectors.cpp", "api.cpp", "hlocal.hip", "plane_tl.hip", "zgemm.hip", "zgemm64.hip", "zgemm32.hip", "aux_kernels.hip",
            "subspace_eig.hip", "potential.hip", "noalloc.hip", "gamma_kernels.hip", "kb_device.hip", "dense.cpp", "davidson.cpp", "batch.cpp", "server.cpp",
            "memory_estimate.cpp"]
 

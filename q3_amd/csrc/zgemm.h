@@ -23,4 +23,12 @@ bool zgemm64_aligned(const void* A, const void* B, const void* C, const void* wo
 hipError_t zgemm64(int tile, int split, int opa, int m, int n, int k, double alpha, const void* A, long lda, const void* B,
                    long ldb, double beta, void* C, long ldc, void* work, size_t work_bytes, hipStream_t st);
 
+// The FP32 products (zgemm32.hip): A^H B with F_D_F_F, A B with F_F_F_D, both with D_D_F_D, of matrices
+// aligned to their elements (zgemm32_takes); tiles 45, 44, 42, 25, 24, 22, 21, 12.
+bool zgemm32_has_tile(int tile);
+bool zgemm32_takes(GemmTypes types, int opa, const void* A, const void* B, const void* C, const void* work);
+hipError_t zgemm32(int tile, int split, GemmTypes types, int opa, int m, int n, int k, double alpha, const void* A,
+                   long lda, const void* B, long ldb, double beta, void* C, long ldc, void* work, size_t work_bytes,
+                   hipStream_t st);
+
 }  // namespace q3x

@@ -1,6 +1,6 @@
-// Complex GEMM on CDNA4 matrix cores with register-staged operands (v_mfma_f32_16x16x4f32, and
-// v_mfma_f64_16x16x4f64 for FP64 matrices that are not 16-byte aligned; the aligned ones go to
-// zgemm64.hip).
+// Complex GEMM on CDNA4 matrix cores with register-staged operands (v_mfma_f64_16x16x4f64,
+// v_mfma_f32_16x16x4f32), for matrices that are not aligned to their elements; the aligned ones go to
+// zgemm64.hip and zgemm32.hip.
 //
 //   C (m x n) = alpha * op(A) * B + beta * C,   op(A) = A (m x k) or A^H (A stored k x m),
 //   alpha, beta real, all matrices column-major interleaved complex.
@@ -339,65 +339,26 @@ hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A
     return hipGetLastError();
 }
 
-// Tile configurations (wave tiles TMW x TNW, K stage KC, minimum waves per SIMD) and how a complex64
-// product picks one.  The table comes from timing every candidate on the H|psi> and Davidson
-// shapes of the 64-atom cell (q3_amd/tune_gemm.py): 2x2 tiles throughout; deep-k A^H B products
-// split K so that the grid is one round of resident workgroups (CUs x occupancy of the kernel): a
-// partial second round costs as much as a full one.
-// Q3X_GEMM_TILE="TMWxTNW/ksplit" overrides the choice (ksplit -1: one round, 0: default).
-enum class Tile { T2x2, T4x2, T2x5, T4x4, T4x5 };
-
+// Which kernel takes a product: zgemm64.hip the FP64 ones and zgemm32.hip the FP32 ones whose matrices are
+// aligned to their elements; this file's 64 x 32 tile the rest (a complex128 pointer that is a multiple
+// of 8 bytes only), A^H B split over one round of resident workgroups.
+// Q3X_GEMM_TILE="TMWxTNW/ksplit" overrides the tile (32 TMW rows by 16 TNW columns) and the K split
+// (<= 0: the built-in choice) of the aligned ones.
 template <typename TA, typename TB, typename TM, typename TC>
-hipError_t zgemm_tile(Tile t, int split, int opa, int m, int n, int k, double alpha, const void* A, long lda,
-                      const void* B, long ldb, double beta, void* C, long ldc, void* work, size_t work_bytes,
-                      hipStream_t st) {
-    switch (t) {
-        case Tile::T2x2:
-            return zgemm_shape<TA, TB, TM, TC, 2, 2, 8, 1>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                           work_bytes, st, split);
-        case Tile::T4x2:
-            return zgemm_shape<TA, TB, TM, TC, 4, 2, 8, 2>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                           work_bytes, st, split);
-        case Tile::T2x5:
-            return zgemm_shape<TA, TB, TM, TC, 2, 5, 8, 2>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                           work_bytes, st, split);
-        case Tile::T4x4:
-            return zgemm_shape<TA, TB, TM, TC, 4, 4, 8, 2>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                           work_bytes, st, split);
-        case Tile::T4x5:
-            return zgemm_shape<TA, TB, TM, TC, 4, 5, 8, 2>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                           work_bytes, st, split);
-    }
-    return hipErrorInvalidValue;
-}
-
-template <typename TA, typename TB, typename TM, typename TC>
-hipError_t zgemm_t(int opa, int m, int n, int k, double alpha, const void* A, long lda, const void* B, long ldb,
-                   double beta, void* C, long ldc, void* work, size_t work_bytes, hipStream_t st) {
+hipError_t zgemm_t(GemmTypes types, int opa, int m, int n, int k, double alpha, const void* A, long lda, const void* B,
+                   long ldb, double beta, void* C, long ldc, void* work, size_t work_bytes, hipStream_t st) {
     if (m <= 0 || n <= 0) return hipSuccess;
-    if constexpr (std::is_same<TM, double>::value) {
-        if (zgemm64_aligned(A, B, C, work)) {
-            int tmw = 0, tnw = 0, sp = 0, tile = 0;
-            const char* cfg = std::getenv("Q3X_GEMM_TILE");
-            if (cfg && std::sscanf(cfg, "%dx%d/%d", &tmw, &tnw, &sp) == 3) tile = 10 * tmw + tnw;
-            if (!zgemm64_has_tile(tile)) tile = sp = 0;
-            return zgemm64(tile, sp, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, st);
-        }
-        return zgemm_shape<TA, TB, TM, TC, 2, 2, 8, 1>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                       work_bytes, st, opa == 1 ? -1 : 0);
-    } else {
-        if (const char* cfg = std::getenv("Q3X_GEMM_TILE")) {
-            int tmw = 0, tnw = 0, sp = 0;
-            if (std::sscanf(cfg, "%dx%d/%d", &tmw, &tnw, &sp) == 3) {  // sp: -1 one round, 0 default, > 0 fixed
-                const Tile t = tmw == 4 ? (tnw == 2 ? Tile::T4x2 : tnw == 4 ? Tile::T4x4 : Tile::T4x5)
-                                        : (tnw == 5 ? Tile::T2x5 : Tile::T2x2);
-                return zgemm_tile<TA, TB, TM, TC>(t, sp, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                  work_bytes, st);
-            }
-        }
-        return zgemm_tile<TA, TB, TM, TC>(Tile::T2x2, opa == 1 ? -1 : 0, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                          work_bytes, st);
+    constexpr bool fp64 = std::is_same<TM, double>::value;
+    if (fp64 ? zgemm64_aligned(A, B, C, work) : zgemm32_takes(types, opa, A, B, C, work)) {
+        int tmw = 0, tnw = 0, sp = 0, tile = 0;
+        const char* cfg = std::getenv("Q3X_GEMM_TILE");
+        if (cfg && std::sscanf(cfg, "%dx%d/%d", &tmw, &tnw, &sp) == 3) tile = 10 * tmw + tnw;
+        if (!(fp64 ? zgemm64_has_tile(tile) : zgemm32_has_tile(tile))) tile = sp = 0;
+        return fp64 ? zgemm64(tile, sp, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, st)
+                    : zgemm32(tile, sp, types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, st);
     }
+    return zgemm_shape<TA, TB, TM, TC, 2, 2, 8, 1>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes,
+                                                   st, opa == 1 ? -1 : 0);
 }
 
 }  // namespace
@@ -407,19 +368,19 @@ hipError_t zgemm(GemmTypes types, int opa, int m, int n, int k, double alpha, co
                  hipStream_t st) {
     switch (types) {
         case GemmTypes::D_D_D_D:
-            return zgemm_t<double, double, double, double>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+            return zgemm_t<double, double, double, double>(types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
                                                            work_bytes, st);
         case GemmTypes::F_D_F_F:
-            return zgemm_t<float, double, float, float>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+            return zgemm_t<float, double, float, float>(types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
                                                         work_bytes, st);
         case GemmTypes::F_F_F_D:
-            return zgemm_t<float, float, float, double>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+            return zgemm_t<float, float, float, double>(types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
                                                         work_bytes, st);
         case GemmTypes::D_D_F_D:
-            return zgemm_t<double, double, float, double>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+            return zgemm_t<double, double, float, double>(types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
                                                           work_bytes, st);
         case GemmTypes::F_F_F_F:
-            return zgemm_t<float, float, float, float>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+            return zgemm_t<float, float, float, float>(types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
                                                        work_bytes, st);
     }
     return hipErrorInvalidValue;

@@ -21,11 +21,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstdint>
 #include <iterator>
 
 #include "zgemm.h"
+#include "zgemm_split.h"
 
 namespace q3x {
 namespace {
@@ -205,49 +205,6 @@ __global__ void __launch_bounds__(256, MINW)
     }
 }
 
-// C = alpha * (sum of the partials) + beta * C.  Four threads an output, each summing a quarter of
-// the K chunks in order with eight loads ahead of their adds, then the quarters in order.
-__global__ void __launch_bounds__(256) splitk_reduce64(int m, long total, int ksplit, const double2* __restrict__ work,
-                                                       double2* __restrict__ C, long ldc, double alpha, double beta) {
-    __shared__ double2 part[3][64];
-    const int q = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const long idx = static_cast<long>(blockIdx.x) * 64 + l;
-    const int per = (ksplit + 3) / 4;
-    int z = q * per;
-    const int z1 = min(ksplit, z + per);
-    double2 s = {0.0, 0.0};
-    if (idx < total) {
-        const double2* w = work + idx;
-        for (; z + 8 <= z1; z += 8) {
-            double2 v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = w[(z + u) * total];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) s.x += v[u].x, s.y += v[u].y;
-        }
-        if (z < z1) {
-            double2 v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = w[min(z + u, z1 - 1) * total];
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (z + u < z1) s.x += v[u].x, s.y += v[u].y;
-        }
-    }
-    if (q > 0) part[q - 1][l] = s;
-    __syncthreads();
-    if (q > 0 || idx >= total) return;
-#pragma unroll
-    for (int u = 0; u < 3; ++u) s.x += part[u][l].x, s.y += part[u][l].y;
-    double2* c = C + idx % m + idx / m * ldc;
-    double2 out = {alpha * s.x, alpha * s.y};
-    if (beta != 0.0) {
-        out.x += beta * c->x;
-        out.y += beta * c->y;
-    }
-    *c = out;
-}
-
 struct Problem {
     int opa, m, n, k;
     double alpha;
@@ -263,72 +220,15 @@ struct Problem {
     hipStream_t st;
 };
 
-// Workgroup tiles: 32 r rows by 16 c columns under the number 10 r + c, K stage KC, workgroups resident
-// on a CU (registers and LDS), and the rate of a product that fills the chip, TF/s.
-struct Tile {
-    int id, bm, bn, kc, resident;
-    double rate;
-};
+// The tiles with their measured rates (4096^3: 72.6 TF/s with the two largest, against 61 and 50 TF/s for
+// A B and A^H B by the register-staged kernel this took over from, and 76 for the vendor's).  What the
+// model of them decides, ms before -> after: overlap 256 x 160 x 51,627 0.349 -> 0.262 (64 x 80, 96
+// splits: three full workgroups per CU), update 51,627 x 160 x 256 0.340 -> 0.259 (128 x 32: 160 =
+// 5 x 32 exactly); A^H B 864 x 440 x 80,927 6.50 -> 3.9; A^H B 32 x 48 x 4,607 0.019 -> 0.009, A B
+// 4,607 x 48 x 96 0.026 -> 0.008 (there the small tiles spread the product over more CUs).
 constexpr Tile kTiles[] = {{44, 128, 64, 8, 2, 72.6}, {42, 128, 32, 8, 3, 71.5}, {25, 64, 80, 8, 3, 71.5},
                            {24, 64, 64, 8, 4, 72.0},  {23, 64, 48, 16, 2, 69.0}, {22, 64, 32, 16, 3, 67.5},
                            {21, 64, 16, 16, 3, 61.5}, {12, 32, 32, 16, 4, 62.5}};
-
-// Which tile and K split a product takes: the pair with the least time by a model of one CU's MFMA,
-// which is what the kernel is bound by (4096^3: 72.6 TF/s with the two largest tiles, against 61 and
-// 50 TF/s for A B and A^H B by the register-staged kernel it took over from, and 76 for the vendor's).
-//   - a CU runs c = ceil(tiles x splits / CUs) workgroups; its MFMA take c x stages x `mfma`,
-//   - a workgroup alone needs `alone` per stage (the barrier and the fragment reads are not hidden,
-//     and below 0.55 us the copy of the next stage is not either), resident ones overlap,
-//   - each round of resident workgroups costs a prologue and an epilogue, and a split product the
-//     traffic and launch of its reduction.
-// The constants are measured (one workgroup per CU: 1.06 us a stage at 64 x 64 x 8 against 0.89 of
-// MFMA, 1.31 at 64 x 80 x 8 against 1.12, 0.56 at 32 x 32 x 16 against 0.45).  What it decides, ms
-// before -> after: overlap 256 x 160 x 51,627 0.349 -> 0.262 (64 x 80, 96 splits: three full
-// workgroups per CU), update 51,627 x 160 x 256 0.340 -> 0.259 (128 x 32: 160 = 5 x 32 exactly);
-// A^H B 864 x 440 x 80,927 6.50 -> 3.9; A^H B 32 x 48 x 4,607 0.019 -> 0.009, A B 4,607 x 48 x 96
-// 0.026 -> 0.008 (there the small tiles spread the product over more CUs).
-// only: 0, or the one tile to consider.
-struct Choice {
-    int tile, split;
-};
-Choice choose(int only, int opa, int m, int n, int k, size_t work_bytes, int cus) {
-    Choice best{24, 1};
-    double least = 0.0;
-    for (const Tile& t : kTiles) {
-        if (only != 0 && t.id != only) continue;
-        const long tiles = static_cast<long>((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-        const double mfma = 8e-6 * t.bm * t.bn * t.kc * cus / t.rate;
-        const double alone = std::max(mfma + 0.17, 0.55);
-        const long most = opa == 1 ? std::min<long>(k / (2 * t.kc), work_bytes / (16ull * m * n)) : 1;
-        for (int fill = 0; fill <= 12; ++fill) {  // 0: no split; else about fill / 2 + 1/2 workgroups per CU
-            long ks = fill == 0 ? 1 : std::min(most, static_cast<long>((fill + 1) / 2) * cus / tiles);
-            if (fill > 0 && ks < 2) continue;
-            if (fill % 2 == 0 && ks >= 8) ks -= ks % 8;  // whole rounds of the XCDs
-            const long stages = ((k + ks - 1) / ks + t.kc - 1) / t.kc;
-            const long c = (tiles * ks + cus - 1) / cus, rounds = (c + t.resident - 1) / t.resident;
-            double us = std::max(c * stages * mfma, rounds * stages * alone) + 2.5 * rounds;
-            if (ks >= 8 && ks % 8) us *= 1.04;
-            if (ks > 1) us += 5.0 + 32e-6 * m * n * ks / 4.0;
-            if (least == 0.0 || us < least) {
-                least = us;
-                best = {t.id, static_cast<int>(ks)};
-            }
-        }
-    }
-    return best;
-}
-
-int cu_count() {
-    static std::atomic<int> cached{0};  // of the first device used; same value from any thread
-    int n = cached.load();
-    if (n == 0) {
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached.store(n);
-    }
-    return n;
-}
 
 template <int OPA, int TM, int TN, int WM, int WN, int KC, int MINW>
 hipError_t launch(const Problem& g, int split) {
@@ -353,8 +253,8 @@ hipError_t launch(const Problem& g, int split) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || ksplit == 1) return e;
     const long total = static_cast<long>(g.m) * g.n;
-    hipLaunchKernelGGL(splitk_reduce64, dim3(static_cast<unsigned>((total + 63) / 64)), dim3(256), 0, g.st, g.m, total,
-                       ksplit, g.work, g.C, g.ldc, g.alpha, g.beta);
+    hipLaunchKernelGGL((splitk_sum<double2, double2>), dim3(static_cast<unsigned>((total + 63) / 64)), dim3(256), 0,
+                       g.st, g.m, total, ksplit, g.work, g.C, g.ldc, g.alpha, g.beta);
     return hipGetLastError();
 }
 
@@ -389,7 +289,8 @@ hipError_t zgemm64(int tile, int split, int opa, int m, int n, int k, double alp
     const Problem g{opa, m, n, k, alpha, static_cast<const double2*>(A), lda, static_cast<const double2*>(B), ldb, beta,
                     static_cast<double2*>(C), ldc, static_cast<double2*>(work), work_bytes, st};
     if (tile == 0 || split <= 0) {
-        const Choice c = choose(tile, opa, m, n, k, work ? work_bytes : 0, cu_count());
+        const long most = opa == 1 && work ? static_cast<long>(work_bytes / (16ull * m * n)) : 1;
+        const Choice c = choose(kTiles, tile, 1, most, 16, m, n, k, cu_count());
         tile = c.tile;
         split = c.split;
     }

@@ -1,9 +1,9 @@
-"""Tile tuner for the complex MFMA GEMM (zgemm.hip).
+"""Tile tuner for the complex MFMA GEMM (zgemm64.hip, zgemm32.hip).
 
 Times every tile configuration the library is built with (and a few K splits for the deep-k A^H B
 products; a tile TMWxTNW covers 32 TMW rows and 16 TNW complex columns per workgroup) on the products of H|psi> and block Davidson for a given plane-wave
 count, band count and projector count, and prints the fastest per shape class and precision.
-The library's built-in choices (the cost model of zgemm64.hip, the complex64 table of zgemm.hip)
+The library's built-in choices (the cost model of zgemm_split.h)
 were fitted to what this printed for the 64-atom Si cell (npw 51,627, 160 bands, 256 projectors); Q3X_GEMM_TILE="TMWxTNW/ksplit" forces one
 configuration at run time, which is how this script measures the candidates.
 
@@ -19,7 +19,7 @@ import time
 import numpy as np
 
 TILES = {"fp64": ["4x4", "4x2", "2x5", "2x4", "2x3", "2x2", "2x1", "1x2"],  # zgemm64.hip
-         "fp32": ["2x2", "4x2", "2x5", "4x4", "4x5"]}                          # zgemm.hip
+         "fp32": ["4x5", "4x4", "4x2", "2x5", "2x4", "2x2", "2x1", "1x2"]}         # zgemm32.hip
 SPLITS = [-1, 0, 64, 128]
 
 
