@@ -79,7 +79,7 @@ __host__ __device__ constexpr int plane_tw_entries(bool fp64, int a, int b) {
 // per CU need four (128 registers); the radix-15/16 complex64 shapes need more and get two
 constexpr int plane_tl_min_waves(bool fp64, int a) { return fp64 || a > 12 ? 2 : 4; }
 
-// DENS: the charge density in place of the sandwich (FP64, plane in LDS).  Workgroup (z, g) =
+// DENS = 1: the charge density in place of the sandwich (FP64, plane in LDS).  Workgroup (z, g) =
 // (blockIdx.x mod n3, blockIdx.x / n3) runs the backward transforms of columns [g per, g per + per)
 // of plane z and adds w_re Re(f)^2 + w_im Im(f)^2 of each into its own partial plane in dens.part,
 // which no other workgroup touches: value (row group, sub-pass, j) of a lane at
@@ -91,6 +91,7 @@ struct PlaneDensity {
     const double2* wts;  // (w_re, w_im) per column
     double* part;
     int per;             // columns per workgroup
+    double* rho;         // DENS = 2 (one column per workgroup): where to add the values instead
 };
 constexpr int plane_part_size(int a, int b) {
     const int gr = plane_group_rows(a, b);
@@ -106,7 +107,7 @@ constexpr int plane_part_size(int a, int b) {
 // 3.37 ms.
 __host__ __device__ constexpr int plane_quarter(int a) { return (a + 3) / 4; }
 
-template <typename T, int A, int B, bool PG, bool QU, bool DENS = false>
+template <typename T, int A, int B, bool PG, bool QU, int DENS = 0>
 __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
                                   plane_tl_min_waves(sizeof(T) == 8, A)) plane_tl(HLocalArgs a, const T* __restrict__ vplane,
                                                  cx<T>* __restrict__ zbuf, const cx<T>* __restrict__ twg, int lc,
@@ -389,8 +390,13 @@ __global__ void __launch_bounds__(plane_tl_max_threads(sizeof(T) == 8, A * B),
                     if constexpr (DENS) {
                         const double2 w = dens.wts[q];
 #pragma unroll
-                        for (int j = 0; j < B; ++j)
-                            part[(sp * B + j) * 64] = vv[sp][j] + (w.x * u[j].x * u[j].x + w.y * u[j].y * u[j].y);
+                        for (int j = 0; j < B; ++j) {
+                            const double d = w.x * u[j].x * u[j].x + w.y * u[j].y * u[j].y;
+                            if constexpr (DENS == 2)
+                                atomicAdd(dens.rho + (static_cast<long>(k1 + A * j) * N + r0 + g) * a.p3.n + z, d);
+                            else
+                                part[(sp * B + j) * 64] = vv[sp][j] + d;
+                        }
                         continue;
                     }
 #pragma unroll
@@ -949,21 +955,39 @@ size_t plane_density_workspace(int n, int n3, const PlaneTlConfig& c, int nvec, 
     return 0;
 }
 
-template <int A, int B, bool QU>
-static hipError_t launch_density_planes(const HLocalArgs& a, const cx<double>* zbuf, const PlaneTlConfig& c, int nvec,
-                                       const double* wts, double* part, int groups, double* rho, hipStream_t st) {
+// Calls of few points are as long as their launches: there the workgroups, of one column each, add to rho
+// themselves instead of leaving partials to density_reduce.  Microseconds a call, direct against
+// reduced: 24^3 with 1, 5 and 12 columns 17.4 / 20.2, 16.6 / 19.9, 23.3 / 26.4; 30^3 with 5 20.0 / 22.0;
+// 45^3 with 1 18.6 / 18.8, with 2 24.8 / 19.5 (the strided adds grow with the box).
+constexpr bool density_direct(long points, int per, int nvec) {
+    return per == 1 && points <= 50000 && points * nvec <= 170000;
+}
+
+template <int A, int B, bool QU, int DENS>
+static hipError_t launch_density_kernel(const HLocalArgs& a, const cx<double>* zbuf, const PlaneTlConfig& c, int nvec,
+                                        int groups, const PlaneDensity& d, hipStream_t st) {
     static std::atomic<bool> raised{false};
     if (!raised) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&plane_tl<double, A, B, false, QU, true>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&plane_tl<double, A, B, false, QU, DENS>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
         raised = true;
     }
+    hipLaunchKernelGGL((plane_tl<double, A, B, false, QU, DENS>), dim3(a.p3.n * groups), dim3(c.threads), c.lds, st, a,
+                       nullptr, const_cast<cx<double>*>(zbuf), static_cast<const cx<double>*>(a.twp), c.lc, c.lr,
+                       c.row_waves, a.p3.n * nvec, nullptr, d);
+    return hipGetLastError();
+}
+
+template <int A, int B, bool QU>
+static hipError_t launch_density_planes(const HLocalArgs& a, const cx<double>* zbuf, const PlaneTlConfig& c, int nvec,
+                                       const double* wts, double* part, int groups, double* rho, hipStream_t st) {
     const int n3 = a.p3.n, per = (nvec + groups - 1) / groups;
-    hipLaunchKernelGGL((plane_tl<double, A, B, false, QU, true>), dim3(n3 * groups), dim3(c.threads), c.lds, st, a, nullptr,
-                       const_cast<cx<double>*>(zbuf), static_cast<const cx<double>*>(a.twp), c.lc, c.lr, c.row_waves,
-                       n3 * nvec, nullptr, PlaneDensity{reinterpret_cast<const double2*>(wts), part, per});
-    const hipError_t e = hipGetLastError();
+    const PlaneDensity d{reinterpret_cast<const double2*>(wts), part, per, rho};
+    // (a flag read by one kernel for both made it 12% slower at 96^3)
+    if (A * B <= 64 && density_direct(static_cast<long>(A * B) * (A * B) * n3, per, nvec))
+        return launch_density_kernel<A, B, QU, A * B <= 64 ? 2 : 1>(a, zbuf, c, nvec, groups, d, st);
+    const hipError_t e = launch_density_kernel<A, B, QU, 1>(a, zbuf, c, nvec, groups, d, st);
     if (e != hipSuccess) return e;
     constexpr int psize = plane_part_size(A, B), gr = plane_group_rows(A, B);
     hipLaunchKernelGGL(density_reduce, dim3(psize / 32, (n3 + 31) / 32), dim3(256), 0, st, A * B, A, B, gr,
