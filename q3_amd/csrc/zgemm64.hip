@@ -289,7 +289,9 @@ hipError_t zgemm64(int tile, int split, int opa, int m, int n, int k, double alp
     const Problem g{opa, m, n, k, alpha, static_cast<const double2*>(A), lda, static_cast<const double2*>(B), ldb, beta,
                     static_cast<double2*>(C), ldc, static_cast<double2*>(work), work_bytes, st};
     if (tile == 0 || split <= 0) {
-        const long most = opa == 1 && work ? static_cast<long>(work_bytes / (16ull * m * n)) : 1;
+        // A B splits too: of few rows and columns and a long k it would else run on a few CUs (32 x 32 x 51,627
+        // 2,057 -> 18 us, 160 x 160 x 51,627 2,074 -> 176 us, 320 x 160 x 320 15.5 -> 9.7 us)
+        const long most = work ? static_cast<long>(work_bytes / (16ull * m * n)) : 1;
         const Choice c = choose(kTiles, tile, 1, most, 16, m, n, k, cu_count());
         tile = c.tile;
         split = c.split;
