@@ -11,8 +11,8 @@
 // same count as a complex GEMM.  Conjugation of op(A) = A^H is folded into the LDS load; B' is
 // written to LDS (complex64) or derived from B at the fragment read (FP64).
 //
-// Workgroup tile: up to 128 rows x 80 complex columns, 4 wave64s in a 2x2 layout, each wave
-// up to 4 x 5 MFMA 16x16 tiles; K staged through double-buffered LDS in chunks of 8 complex.
+// Workgroup tile: 64 rows x 32 complex columns, or for large FP64 products 128 x 32 or 64 x 80; 4 wave64s
+// in a 2x2 layout; K staged through double-buffered LDS in chunks of 8 complex.
 // Tall-skinny products (k >> m, n: projector overlaps, subspace Gram blocks) split
 // K over the grid's z dimension into a workspace and are summed in a fixed order by a
 // second kernel, so results do not depend on scheduling.
@@ -21,6 +21,7 @@
 #include "zgemm.h"
 
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <type_traits>
@@ -50,7 +51,7 @@ struct Mma<float> {
     }
 };
 
-constexpr int KC_DEFAULT = 8;  // complex k per LDS stage (16 real k, four MFMA k-steps)
+constexpr int KC = 8;  // complex k per LDS stage (16 real k, four MFMA k-steps)
 
 // Workgroup: 2 x 2 wave64s; each wave owns TMW x TNW MFMA tiles of 16 x 16 real, so the
 // workgroup tile is BM = 32 TMW rows by BN = 32 TNW real columns (16 TNW complex columns).
@@ -59,7 +60,7 @@ constexpr int KC_DEFAULT = 8;  // complex k per LDS stage (16 real k, four MFMA 
 // barrier per stage orders everything.  LDS rows are padded so that the k-contiguous
 // operand stores (threads walking k) and the fragment reads (lanes walking rows / columns)
 // both spread over the banks.
-template <typename TA, typename TB, typename TM, typename TC, int OPA, int TMW, int TNW, int KC, int MINW>
+template <typename TA, typename TB, typename TM, typename TC, int OPA, int TMW, int TNW, int MINW>
 __global__ void __launch_bounds__(256, MINW) zgemm_kernel(int m, int n, int k, int kchunk, const TA* __restrict__ A,
                                                     long lda, const TB* __restrict__ B, long ldb, TC* __restrict__ C,
                                                     long ldc, double alpha, double beta, TM* __restrict__ work,
@@ -269,16 +270,15 @@ __global__ void splitk_reduce(int m, int n, int ksplit, const TM* __restrict__ w
     C[o] = static_cast<TC>(out);
 }
 
-template <typename TA, typename TB, typename TM, typename TC, int TMW, int TNW, int KC = KC_DEFAULT, int MINW = 1>
-hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A, long lda, const void* B, long ldb,
-                       double beta, void* C, long ldc, void* work, size_t work_bytes, hipStream_t st,
-                       int force_split = 0) {
+template <typename TA, typename TB, typename TM, typename TC, int OPA, int TMW, int TNW, int MINW>
+hipError_t zgemm_shape(int m, int n, int k, double alpha, const void* A, long lda, const void* B, long ldb,
+                       double beta, void* C, long ldc, void* work, size_t work_bytes, hipStream_t st) {
     constexpr int BM = 32 * TMW, BNC = 16 * TNW;
     const int tm = (m + BM - 1) / BM, tn = (n + BNC - 1) / BNC;
     const long tiles = static_cast<long>(tm) * tn;
     int ksplit = 1;
     const long by_ws = work ? static_cast<long>(work_bytes / (2ull * m * n * sizeof(TM))) : 1;
-    if (force_split < 0 && work && k > 0) {
+    if (OPA == 1 && work && k > 0) {
         // fill one round of the GPU: workgroups resident at once = CUs x blocks per CU of this kernel
         static std::atomic<int> slots_cached{0};  // per kernel instantiation; same value from any thread
         int slots = slots_cached.load();
@@ -287,14 +287,12 @@ hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A
             (void)hipGetDevice(&dev);
             (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
             (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, reinterpret_cast<const void*>(&zgemm_kernel<TA, TB, TM, TC, 1, TMW, TNW, KC, MINW>), 256, 0);
+                &per_cu, reinterpret_cast<const void*>(&zgemm_kernel<TA, TB, TM, TC, OPA, TMW, TNW, MINW>), 256, 0);
             slots = std::max(1, cus * std::max(1, per_cu));
             slots_cached.store(slots);
         }
         const long by_k = std::max(1, k / 128);  // at least 128 complex k per split
         ksplit = static_cast<int>(std::max(1L, std::min(std::min(slots / tiles, by_k), by_ws)));
-    } else if (force_split > 0 && work) {
-        ksplit = static_cast<int>(std::max(1L, std::min<long>(force_split, by_ws)));
     } else if (k > 0 && tiles < 512 && work) {
         long want = (1024 + tiles - 1) / tiles;
         long by_k = (k + 511) / 512;  // at least 512 complex k per split
@@ -306,31 +304,25 @@ hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A
     // overlap) and keep the plain order.
     // The chunk count stays that multiple of 8 after the chunk length is rounded up to KC: chunks
     // past the end of K are empty and add zero partials.
-    const bool want_xmap = sizeof(TM) == 8 && ksplit >= 8;
-    const bool keep8 = want_xmap && force_split <= 0;
-    if (keep8) ksplit -= ksplit % 8;
+    const bool by_xcd = sizeof(TM) == 8 && ksplit >= 8;
+    if (by_xcd) ksplit -= ksplit % 8;
     int kchunk = (k + ksplit - 1) / ksplit;
     kchunk = ((kchunk + KC - 1) / KC) * KC;
     if (kchunk == 0) kchunk = KC;
-    if (!keep8) ksplit = k > 0 ? (k + kchunk - 1) / kchunk : 1;
-    int xmap = want_xmap && ksplit % 8 == 0 ? 1 : 0;
+    if (!by_xcd) ksplit = k > 0 ? (k + kchunk - 1) / kchunk : 1;
+    int xmap = by_xcd ? 1 : 0;
     dim3 grid(tm, tn, ksplit);
     // A B without a split (the projector update Hpsi += beta W): the column tiles of a row block
     // run one after another on one XCD (xmap 2), so each row block of A is fetched once: the
     // complex64 update of 51,627 x 160 x 256 reads 286 MB instead of 802 MB in the same time
-    if (opa == 0 && ksplit == 1 && tn > 1) {
+    if (OPA == 0 && ksplit == 1 && tn > 1) {
         xmap = 2;
         grid.x = (tm + 7) / 8 * 8;
     }
     TM* w = ksplit > 1 ? static_cast<TM*>(work) : nullptr;
-    if (opa == 0)
-        hipLaunchKernelGGL((zgemm_kernel<TA, TB, TM, TC, 0, TMW, TNW, KC, MINW>), grid, dim3(256), 0, st, m, n, k, kchunk,
-                           static_cast<const TA*>(A), lda, static_cast<const TB*>(B), ldb, static_cast<TC*>(C), ldc,
-                           alpha, beta, w, xmap);
-    else
-        hipLaunchKernelGGL((zgemm_kernel<TA, TB, TM, TC, 1, TMW, TNW, KC, MINW>), grid, dim3(256), 0, st, m, n, k, kchunk,
-                           static_cast<const TA*>(A), lda, static_cast<const TB*>(B), ldb, static_cast<TC*>(C), ldc,
-                           alpha, beta, w, xmap);
+    hipLaunchKernelGGL((zgemm_kernel<TA, TB, TM, TC, OPA, TMW, TNW, MINW>), grid, dim3(256), 0, st, m, n, k, kchunk,
+                       static_cast<const TA*>(A), lda, static_cast<const TB*>(B), ldb, static_cast<TC*>(C), ldc, alpha,
+                       beta, w, xmap);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || ksplit == 1) return e;
     const long total = 2L * m * n;
@@ -340,8 +332,13 @@ hipError_t zgemm_shape(int opa, int m, int n, int k, double alpha, const void* A
 }
 
 // Which kernel takes a product: zgemm64.hip the FP64 ones and zgemm32.hip the FP32 ones whose matrices are
-// aligned to their elements; this file's 64 x 32 tile the rest (a complex128 pointer that is a multiple
-// of 8 bytes only), A^H B split over one round of resident workgroups.
+// aligned to their elements; this file's the rest (a complex128 pointer that is a multiple of 8 bytes
+// only), A^H B split over one round of resident workgroups.  Its 64 x 32 tile, but for FP64 products
+//   - A B where the rounds of 256 CUs that its 128 x 32 tiles take, of 1.75 times the length, are shorter
+//     together: 10,000 x 160 x 256 89 -> 82 us (7/4 x 2 rounds for 4), 51,627 x 160 x 256 334 -> 301; of
+//     20,000 x 160 x 256 the 64 x 32 tiles take 151 us (7 rounds) and these 156 (7/4 x 4);
+//   - A^H B that fill 64 x 80 tiles, of 3e8 multiply-adds or more: 320 x 80 x 51,627 320 -> 228 us,
+//     256 x 160 x 12,000 103 -> 98; below it 256 x 160 x 4,607 takes 51 us with 64 x 32 tiles and 53.
 // Q3X_GEMM_TILE="TMWxTNW/ksplit" overrides the tile (32 TMW rows by 16 TNW columns) and the K split
 // (<= 0: the built-in choice) of the aligned ones.
 template <typename TA, typename TB, typename TM, typename TC>
@@ -357,8 +354,20 @@ hipError_t zgemm_t(GemmTypes types, int opa, int m, int n, int k, double alpha, 
         return fp64 ? zgemm64(tile, sp, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, st)
                     : zgemm32(tile, sp, types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, st);
     }
-    return zgemm_shape<TA, TB, TM, TC, 2, 2, 8, 1>(opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes,
-                                                   st, opa == 1 ? -1 : 0);
+    if constexpr (fp64) {
+        // (an unsplit A B rounds its row tiles up to a multiple of 8)
+        auto rounds = [&](int rows) { return ((m + rows - 1) / rows + 7L) / 8 * 8 * ((n + 31) / 32) / 256.0; };
+        if (opa == 0 && m > 64 && n > 32 && 1.75 * std::ceil(rounds(128)) < std::ceil(rounds(64)))
+            return zgemm_shape<TA, TB, TM, TC, 0, 4, 2, 2>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes,
+                                                           st);
+        if (opa == 1 && m > 64 && n % 80 == 0 && static_cast<double>(m) * n * k >= 3e8)
+            return zgemm_shape<TA, TB, TM, TC, 1, 2, 5, 2>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes,
+                                                           st);
+    }
+    return opa == 0 ? zgemm_shape<TA, TB, TM, TC, 0, 2, 2, 1>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+                                                              work_bytes, st)
+                    : zgemm_shape<TA, TB, TM, TC, 1, 2, 2, 1>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
+                                                              work_bytes, st);
 }
 
 }  // namespace
