@@ -23,6 +23,7 @@
 // and transforms are complex64).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "fft_lds.h"
@@ -206,11 +207,17 @@ size_t hlocal_lds_bytes(const HLocalArgs& a, bool fp32, int which) {
 }
 
 template <typename T>
-hipError_t launch_hlocal_t(const HLocalArgs& a, const T* vplane, void* zbuf, const double* psi, long ldpsi,
+hipError_t launch_hlocal_t(HLocalArgs a, const T* vplane, void* zbuf, const double* psi, long ldpsi,
                            double* hpsi, long ldh, int nvec, hipStream_t st, hipEvent_t* marks,
                            const PlaneTlConfig* tl, void* pglob, const StickTlConfig* tz) {
     if (marks) (void)hipEventRecord(marks[0], st);
     const bool fp32 = sizeof(T) == 4;
+    // Generic z-sticks of a call that would leave CUs idle: fewer to a workgroup (whole rounds of its four
+    // wavefronts), so that it is one round of 256 workgroups.  A 50 x 30 x 30 box has 177 sticks of 50, three
+    // workgroups a band: H|psi> of 1 and 8 bands 28.0 -> 16.6 and 31.8 -> 20.0 us; 192 x 32 x 32, 8 bands 50.9 ->
+    // 42.8 us.  (Two rounds of fewer sticks made 16 bands of 25 x 36 x 36 24.6 -> 27.5 us.)
+    a.sticks_per_block = static_cast<int>(
+        std::min<long>(a.sticks_per_block, (static_cast<long>(a.nst) * nvec + 1023) / 1024 * 4));
     const int nsb_blocks = (a.nst + a.sticks_per_block - 1) / a.sticks_per_block;
     dim3 g1(nsb_blocks, nvec);
     const size_t lds_z = hlocal_lds_bytes(a, fp32, 0);

@@ -49,7 +49,10 @@ struct BasisData {
 // plane kernels are built for, the order that puts those two into the plane: a 72 x 36 x 36 box runs
 // its square 36 x 36 planes there instead of 72 x 36 planes in the generic kernel (75 x 40 x 40, 39
 // bands: plane stage 188 -> 63 us).  Lengths up to 120, whose planes the generic kernels can hold in
-// LDS too.  i1, i2, i3 below and in the kernels count along axis[0], axis[1], axis[2].
+// LDS too.  The sticks may then have a length without a two-level kernel: H|psi> of 1, 8 and 32 bands in
+// 50 x 30 x 30 25.6, 26.9, 81 -> 16.5, 20.1, 37 us, in 180 x 30 x 30 42.6, 45, 151 -> 19.3, 38, 99.  Slower
+// is a single FP64 band where few planes of 120 do not fit in LDS (18 x 120 x 120 43 -> 48 us; 8 bands
+// 126 -> 65).  i1, i2, i3 below and in the kernels count along axis[0], axis[1], axis[2].
 void transform_axes(const int wave[3], int axis[3]);
 
 // Stick decomposition of one k-point's sphere for the pencil FFT.
