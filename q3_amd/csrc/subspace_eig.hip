@@ -80,10 +80,6 @@ __device__ __forceinline__ double wave_sum(double v) {
     v += dpp_mov<0xB1>(v);
     return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
-// Sums of V values per lane over the wavefront at once (V a power of 2, <= 64): each exchange
-// stage swaps half of the live values with the partner lane and adds, halving V, so V sums
-// cost about log2(64) + V - 1 exchanges instead of 6 V.  On return lane l holds the full sum of
-// value l / (64 / V).
 // Sum of two values over lane pairs l, l ^ 32 (SWAP32) or l ^ 16: the lanes with that bit clear get
 // the sum of a, the others that of b.  A lane swap between the two registers leaves both addends of a
 // lane's sum in that lane, without selects and without an LDS round trip.
@@ -102,6 +98,10 @@ __device__ __forceinline__ double swap_sum(double a, double b) {
            __hiloint2double(static_cast<int>(hi.y), static_cast<int>(lo.y));
 }
 
+// Sums of V values per lane over the wavefront at once (V a power of 2, 2 to 32): each exchange
+// stage swaps half of the live values with the partner lane and adds, halving V, so V sums
+// cost about log2(64) + V - 1 exchanges instead of 6 V.  On return lane l holds the full sum of
+// value l / (64 / V).
 template <int V>
 __device__ __forceinline__ double wave_multi_sum(double (&x)[V], int lane) {
     static_assert(V >= 2 && V <= 32, "at least one value to swap");
@@ -414,9 +414,8 @@ __device__ double column_step(z2* M, int n, int j, double tn, const z2* vn, cons
 // Pass of step k over columns / rows [k+2, n): rank-2 update with (v, q) when tk != 0, then
 // p[c] = tn * (column)^H vn when tn != 0.  Wavefront w takes CB adjacent columns at a time.  The
 // row vectors v, q, vn are the same for every column of the pass, so each lane loads its rows of
-// them into registers once (they share LDS with the matrix, so re-reading them after a column
-// store would be a dependent LDS round trip per column); the CB columns' loads are issued
-// together, and their 2 CB wave reductions run side by side with no branch between them.
+// them into registers once; the CB columns' loads are issued together, and their 2 CB wave
+// reductions run side by side with no branch between them.
 // v, q index rows from k+1; vn and p from k+2.
 template <int RPL, int CB>
 __device__ void fused_pass(z2* M, int n, int k, double tk, const z2* v, const z2* q, double tn, const z2* vn,
@@ -490,11 +489,12 @@ __device__ void fused_pass(z2* M, int n, int k, double tk, const z2* v, const z2
 
 // A (n x n, ld n, full storage, Hermitian up to rounding) -> d (diagonal), beta (sub-diagonal,
 // beta[i] couples i-1 and i), tau (reflectors, kept in A below the sub-diagonal), the real
-// tridiagonal |beta| in eabs and the phases D in phase (T = D Tr D^H).  RPL >= ceil(n / 64).
+// tridiagonal |beta| in eabs and the phases D in phase (T = D Tr D^H).  n > 128 (a matrix whose
+// exchange between workgroups gave up); RPL >= ceil(n / 64).
 template <int RPL>
 __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double* d, z2* beta, double* tau,
                                                            z2* phase, double* eabs) {
-    constexpr int CB = RPL <= 2 ? 4 : (RPL <= 4 ? 2 : 1);
+    constexpr int CB = RPL <= 4 ? 2 : 1;
     extern __shared__ z2 sh[];
     z2* vb0 = sh;
     z2* vb1 = sh + n;
@@ -526,56 +526,46 @@ __global__ __launch_bounds__(kThreads) void tridiag_kernel(z2* A, int n, double*
         sd[i] = 0.0;
     }
     __syncthreads();
-    if (n <= 2) {
-        if (tid == 0) {
-            sd[0] = M[0].x;
-            if (n == 2) {
-                sd[1] = M[3].x;
-                sbeta[1] = M[1];
-            }
-        }
-    } else {
-        // reflector 0 (column 0 needs no update)
-        if (wv == 0) {
-            const double t0 = column_step<RPL>(M, n, 0, 0.0, nullptr, nullptr, 0.0, vb0, sd, sbeta, stau);
-            if ((tid & 63) == 0) tnext = t0;
+    // reflector 0 (column 0 needs no update)
+    if (wv == 0) {
+        const double t0 = column_step<RPL>(M, n, 0, 0.0, nullptr, nullptr, 0.0, vb0, sd, sbeta, stau);
+        if ((tid & 63) == 0) tnext = t0;
+    }
+    __syncthreads();
+    double tk = 0.0, tn = tnext;
+    z2* v = vb1;   // reflector k (not yet defined at k = -1)
+    z2* vn = vb0;  // reflector k+1
+    // Once the trailing block has at most 64 rows, one row per lane covers it: the passes and
+    // column steps drop the second row set, which would only add masked zeros.
+    for (int k = -1; k <= n - 3; ++k) {
+        const bool one_row = n - k - 2 <= 64;
+        if (tk != 0.0 || tn != 0.0) {
+            if (one_row)
+                fused_pass<1, 4>(M, n, k, tk, v, q, tn, vn, p);
+            else
+                fused_pass<RPL, CB>(M, n, k, tk, v, q, tn, vn, p);
         }
         __syncthreads();
-        double tk = 0.0, tn = tnext;
-        z2* v = vb1;   // reflector k (not yet defined at k = -1)
-        z2* vn = vb0;  // reflector k+1
-        // Once the trailing block has at most 64 rows, one row per lane covers it: the passes and
-        // column steps drop the second row set, which would only add masked zeros.
-        for (int k = -1; k <= n - 3; ++k) {
-            const bool one_row = RPL > 1 && n - k - 2 <= 64;
-            if (tk != 0.0 || tn != 0.0) {
-                if (one_row)
-                    fused_pass<1, 4>(M, n, k, tk, v, q, tn, vn, p);
-                else
-                    fused_pass<RPL, CB>(M, n, k, tk, v, q, tn, vn, p);
+        const int len = n - k - 2;
+        if (wv == 0) {  // f = tn vn^H p / 2, q = p - f vn, next column and reflector: one wavefront
+            const int lane = tid & 63;
+            double f = 0.0;
+            if (tn != 0.0) {
+                double part = 0.0;
+                for (int i = lane; i < len; i += 64) part += vn[i].x * p[i].x + vn[i].y * p[i].y;
+                f = 0.5 * tn * wave_sum(part);
+                for (int i = lane; i < len; i += 64) q[i] = {p[i].x - f * vn[i].x, p[i].y - f * vn[i].y};
             }
-            __syncthreads();
-            const int len = n - k - 2;
-            if (wv == 0) {  // f = tn vn^H p / 2, q = p - f vn, next column and reflector: one wavefront
-                const int lane = tid & 63;
-                double f = 0.0;
-                if (tn != 0.0) {
-                    double part = 0.0;
-                    for (int i = lane; i < len; i += 64) part += vn[i].x * p[i].x + vn[i].y * p[i].y;
-                    f = 0.5 * tn * wave_sum(part);
-                    for (int i = lane; i < len; i += 64) q[i] = {p[i].x - f * vn[i].x, p[i].y - f * vn[i].y};
-                }
-                const double tj = one_row ? column_step<1>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau)
-                                          : column_step<RPL>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau);
-                if (lane == 0) tnext = tj;
-            }
-            __syncthreads();
-            tk = tn;
-            tn = tnext;
-            z2* t = v;
-            v = vn;
-            vn = t;
+            const double tj = one_row ? column_step<1>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau)
+                                      : column_step<RPL>(M, n, k + 2, tn, vn, p, f, v, sd, sbeta, stau);
+            if (lane == 0) tnext = tj;
         }
+        __syncthreads();
+        tk = tn;
+        tn = tnext;
+        z2* t = v;
+        v = vn;
+        vn = t;
     }
     __syncthreads();
     for (int i = tid; i < n; i += nt) {
@@ -690,6 +680,20 @@ __device__ double first_reflector(const z2* A, int n, z2* p, z2* pc, z2* v, z2* 
         out.tau[n - 1] = 0.0;
     }
     return t0;
+}
+
+// n <= 2: no reflector.  One wavefront.
+__global__ __launch_bounds__(64) void tridiag_tiny(const z2* __restrict__ A, int n, double* d, z2* beta, double* tau,
+                                                   z2* phase, double* eabs) {
+    __shared__ z2 sbeta[2];
+    const int i = threadIdx.x;
+    if (i < n) {
+        d[i] = A[i + i * n].x;
+        tau[i] = 0.0;
+        beta[i] = sbeta[i] = i == 0 ? z2{0.0, 0.0} : herm_entry(A, n, 1, 0);
+    }
+    __syncthreads();
+    phases_wave(n, sbeta, phase, eabs);
 }
 
 // One workgroup of 8 wavefronts, n <= 128: column w + 8 (CPW - 1 - c) is the c-th of wavefront w and
@@ -975,7 +979,7 @@ __global__ __launch_bounds__(64 * kGridWaves) void tridiag_grid(const z2* __rest
 }
 
 // ---------------------------------------------------------------- 3c. tridiagonalisation over the LDS of many CUs ----
-// Matrices too large for the registers of one XCD (3b).  The same reduction with the matrix spread
+// Matrices too large for the registers of 3b's workgroups.  The same reduction with the matrix spread
 // over the LDS of W workgroups: column j lives in
 // workgroup j mod W (all rows), so the passes run at LDS speed on W CUs instead of at one CU's
 // L2 bandwidth.  Per step: every workgroup updates its own columns and forms its entries of p;
@@ -993,7 +997,7 @@ __global__ __launch_bounds__(64 * kGridWaves) void tridiag_grid(const z2* __rest
 // Each workgroup owns one flag word (flags[32 w], a 128-byte line of its own) and stores the
 // step number there; its first wavefront polls the other W - 1 flags, one per lane.  Stores to
 // separate lines replace W atomic adds to one word, which the memory side serialises: at
-// n = 320 (20 workgroups) a reduction takes 4.8% less time, at n = 640 (64) 15% less.
+// n = 640 (64 workgroups) a reduction takes 15% less time.
 // Release fence, relaxed store, relaxed polls, one acquire fence: each fence pair synchronises
 // through the flag it reads, and no poll pays for an acquire (an agent-scope acquire
 // invalidates cache lines; a seq_cst fence on each side would write back and invalidate twice).
@@ -1265,6 +1269,9 @@ __device__ int sturm_count(int n, const double2* de, double x) {
     for (; i < n; ++i) step(de[i]);
     return static_cast<int>(c);
 }
+
+// Gershgorin interval [gl, gu] of the tridiagonal, its norm bound tn and pivmin; lane-parallel
+// over one wavefront, same result in every lane.
 __device__ void tri_bounds(int n, const double* d, const double* e, double& gl, double& gu, double& tn,
                            double& pivmin) {
     const int lane = threadIdx.x & 63;
@@ -1810,12 +1817,14 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
             *err = hipErrorInvalidValue;
             return -1;
         }
-        // one CU's registers, those of several CUs, the LDS of many CUs; or (n <= 2, and a solve redone
-        // after a wait that gave up) one workgroup on the matrix in L2
-        z2* refl = C;  // where the reflectors end up
+        // one CU's registers, those of several CUs, the LDS of many CUs; or (a solve redone after a wait
+        // that gave up) one workgroup on the matrix in L2
+        z2* refl = T1;  // where the reflectors end up
         bool grid_done = false;
-        if (n >= 3 && n <= kCuMax) {
-            refl = T1;
+        if (n <= 2) {
+            hipLaunchKernelGGL(tridiag_tiny, dim3(1), dim3(64), 0, st, C, n, d, beta, tau, ph, e);
+            refl = C;
+        } else if (n <= kCuMax) {
 #define Q3X_TRC(CP, RP) \
     hipLaunchKernelGGL((tridiag_cu<CP, RP>), dim3(1), dim3(64 * kCuWaves), 0, st, C, n, T1, d, beta, tau, ph, e)
             if (n <= 16) Q3X_TRC(2, 1);
@@ -1824,7 +1833,7 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
             else if (n <= 96) Q3X_TRC(12, 2);
             else Q3X_TRC(16, 2);
 #undef Q3X_TRC
-        } else if (n > kCuMax && n <= kGridMax && multi_wg_ok && n / kGridCols < num_cus_hint) {
+        } else if (n <= kGridMax && multi_wg_ok && n / kGridCols < num_cus_hint) {
             // word 1: the give-up flag; the words of p and of the pivot column lie before it
             unsigned* bar = reinterpret_cast<unsigned*>(base + L.off[B_BAR]);
             u64 *xp = reinterpret_cast<u64*>(base + L.off[B_XP]), *xc = reinterpret_cast<u64*>(base + L.off[B_XC]);
@@ -1849,7 +1858,6 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
 #undef Q3X_TRG
             if (!ok(hipGetLastError())) return -1;
             grid_done = true;
-            refl = T1;
         } else if (n > kGridMax && multi_wg_ok) {
             const long room = static_cast<long>(max_lds / 16) - 5L * n - 16;
             const int ncl = static_cast<int>(std::min<long>(16, room / n));
@@ -1882,20 +1890,19 @@ int subspace_eig(int n, const double* H, long ldh, const double* S, long lds, in
                                        xp, xc, bar, fail);
                     if (!ok(hipGetLastError())) return -1;
                     grid_done = true;
-                    refl = T1;
                 }
             }
         }
 #define Q3X_TRD(R) \
         hipLaunchKernelGGL((tridiag_kernel<R>), dim3(1), dim3(kThreads), tl, st, C, n, d, beta, tau, ph, e)
-        if (refl == T1) {
-        } else if (rows_lane <= 1) Q3X_TRD(1);
-        else if (rows_lane <= 2) Q3X_TRD(2);
-        else if (rows_lane <= 4) Q3X_TRD(4);
-        else if (rows_lane <= 6) Q3X_TRD(6);
-        else if (rows_lane <= 8) Q3X_TRD(8);
-        else if (rows_lane <= 12) Q3X_TRD(12);
-        else Q3X_TRD(16);
+        if (n > kCuMax && !grid_done) {
+            refl = C;
+            if (rows_lane <= 4) Q3X_TRD(4);
+            else if (rows_lane <= 6) Q3X_TRD(6);
+            else if (rows_lane <= 8) Q3X_TRD(8);
+            else if (rows_lane <= 12) Q3X_TRD(12);
+            else Q3X_TRD(16);
+        }
     #undef Q3X_TRD
         if (!ok(hipGetLastError())) return -1;
         stage_done(K_EIG_TRIDIAG);
