@@ -178,7 +178,9 @@ q3x_status q3x_hamiltonian_apply_device(q3x_hamiltonian h, const void* d_psi, vo
  * e^{i(k+G).r} (the unnormalised backward transform).  d_psi: npw x nb complex128 in HBM (with the
  * Gamma trick, the half-sphere blocks: pairs of real bands share one transform); weights: nb
  * host doubles (w_k f_nk / Omega for the reference's rho); d_rho: n1 n2 n3 doubles in HBM,
- * C order (i1, i2, i3), added to (the caller clears it).  Stream-ordered.  FP64.  Needs a box the
+ * C order (i1, i2, i3), added to (the caller clears it).  Stream-ordered.  FP64.  The columns (bands,
+ * or pairs) of a call are summed in a fixed order, except in boxes of at most 50,000 points with at
+ * most 170,000 points x columns, where the result repeats to rounding.  Needs a box the
  * two-level kernels cover with every plane wave inside it (Q3X_ERR_ARGUMENT otherwise). */
 q3x_status q3x_hamiltonian_accumulate_density(q3x_hamiltonian h, const void* d_psi, int nb, const double* weights,
                                               void* d_rho);

@@ -956,9 +956,12 @@ size_t plane_density_workspace(int n, int n3, const PlaneTlConfig& c, int nvec, 
 }
 
 // Calls of few points are as long as their launches: there the workgroups, of one column each, add to rho
-// themselves instead of leaving partials to density_reduce.  Microseconds a call, direct against
-// reduced: 24^3 with 1, 5 and 12 columns 17.4 / 20.2, 16.6 / 19.9, 23.3 / 26.4; 30^3 with 5 20.0 / 22.0;
-// 45^3 with 1 18.6 / 18.8, with 2 24.8 / 19.5 (the strided adds grow with the box).
+// themselves instead of leaving partials to density_reduce; several columns then add in the order in which
+// their workgroups arrive, so such a density repeats to rounding only.  Microseconds a call, direct / reduced,
+// with 1, 3, 5 and 8 columns: 24^3 11.9 / 14.0, 12.5 / 15.6, 13.9 / 17.2, 16.8 / 20.0; 32^3 12.1 / 14.5,
+// 14.6 / 16.8, 17.7 / 19.2, 22.3 / 22.9; 36^3 12.8 / 15.1, 16.4 / 17.3, 21.2 / 20.0, 27.5 / 24.6 (even with 4);
+// 40^3 with 1 and 2 14.3 / 15.1, 17.2 / 16.5; 45^3 with 1 17.8 / 16.7: the strided adds grow with the box.  Past
+// the second limit 24^3 and 30^3 would still gain up to 2 us, for which the ordered sums are not given up.
 constexpr bool density_direct(long points, int per, int nvec) {
     return per == 1 && points <= 50000 && points * nvec <= 170000;
 }
@@ -985,8 +988,10 @@ static hipError_t launch_density_planes(const HLocalArgs& a, const cx<double>* z
     const int n3 = a.p3.n, per = (nvec + groups - 1) / groups;
     const PlaneDensity d{reinterpret_cast<const double2*>(wts), part, per, rho};
     // (a flag read by one kernel for both made it 12% slower at 96^3)
-    if (A * B <= 64 && density_direct(static_cast<long>(A * B) * (A * B) * n3, per, nvec))
-        return launch_density_kernel<A, B, QU, A * B <= 64 ? 2 : 1>(a, zbuf, c, nvec, groups, d, st);
+    if constexpr (density_direct(24L * A * B * A * B, 1, 1)) {  // 24: the shortest stick with a kernel
+        if (density_direct(static_cast<long>(A * B) * (A * B) * n3, per, nvec))
+            return launch_density_kernel<A, B, QU, 2>(a, zbuf, c, nvec, groups, d, st);
+    }
     const hipError_t e = launch_density_kernel<A, B, QU, 1>(a, zbuf, c, nvec, groups, d, st);
     if (e != hipSuccess) return e;
     constexpr int psize = plane_part_size(A, B), gr = plane_group_rows(A, B);
