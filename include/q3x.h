@@ -246,6 +246,10 @@ void q3x_debug_force_barrier_giveups(int count);
  * process) report a non-positive-definite S (zhegv info > n) without solving, so that Davidson's
  * recovery paths (forced collapse, previous eigenvalues kept) can be run on purpose. */
 void q3x_debug_fail_eigensolves(unsigned long long mask);
+/* No counterpart in the reference.  Form of the plane kernel that the prepared k-point's H|psi> takes in the
+ * given precision, for tests: 0 generic, 1 two-level, 2 two-level with the transforms pruned to a sphere
+ * in the outer quarters of the plane; -1 without a prepared k-point. */
+int q3x_debug_plane_form(q3x_hamiltonian h, int precision);
 /* Solves redone on one workgroup since the process started. */
 long q3x_eig_barrier_redos_total(void);
 

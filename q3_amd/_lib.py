@@ -100,6 +100,7 @@ SIGNATURES = {
     "q3x_kpoint_minus_map": (_i, [_p, _p]),
     "q3x_debug_force_barrier_giveups": (None, [_i]),
     "q3x_debug_fail_eigensolves": (None, [ctypes.c_ulonglong]),
+    "q3x_debug_plane_form": (_i, [_p, _i]),
     "q3x_eig_barrier_redos_total": (_l, []),
     "q3x_zgemm": (_i, [_p, ctypes.c_char, _i, _i, _i, _d, _p, _l, _p, _l, _d, _p, _l, _i]),
     "q3x_device_alloc": (_i, [_p, _ul, _pp]),

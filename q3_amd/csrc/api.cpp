@@ -676,6 +676,12 @@ void q3x_debug_force_barrier_giveups(int count) { force_barrier_giveups(count); 
 
 void q3x_debug_fail_eigensolves(unsigned long long mask) { fail_eigensolves(mask); }
 
+int q3x_debug_plane_form(q3x_hamiltonian h, int precision) {
+    if (!h || !h->kp) return -1;
+    const PlaneTlConfig& tl = precision == Q3X_MIXED ? h->tl32 : h->tl64;
+    return !tl.ok ? 0 : tl.quarters ? 2 : 1;
+}
+
 long q3x_eig_barrier_redos_total(void) { return barrier_redos_total(); }
 
 q3x_status q3x_device_alloc(q3x_context ctx, unsigned long bytes, void** out) {

@@ -1,12 +1,14 @@
 """The plane kernels' pruned form (occupied sticks and columns in the outer quarters of the plane) and the
 general one, on either side of the line: cells whose sphere reaches into the inner blocks of the box
-(k outside the first zone shifts it there) and cells whose sphere does not, against the generic kernels,
-FP64 to rounding and mixed to 2e-6; the density of both against numpy."""
+(k outside the first zone shifts it there) and cells whose sphere does not.  The form that runs is the one that
+the sphere asks for; H psi and the density of both against numpy, and against the generic kernels where those
+hold the plane, FP64 to rounding and mixed to 2e-6."""
 import numpy as np
 import pytest
 
 from q3_amd import FP64, MIXED, PlanewaveHamiltonianApplicator
 from q3_amd import workloads as W
+from q3_amd._lib import Q3XError, lib
 from q3_amd.planewave import Crystal, PlanewaveBasis
 from tests.helpers import rel_err
 
@@ -40,30 +42,43 @@ def test_both_sides_of_the_line(gpu_context, monkeypatch, n, k):
     inside = not (_inner(n, i1) or _inner(n, i2))
     print(f"n={n} k={k}: {'pruned' if inside else 'general'}", flush=True)
     psi = W.random_psi(kp.kinetic_energy_squared, 3, seed=n)
-    out = []
-    for generic in (False, True):
-        if generic:
-            monkeypatch.setenv("Q3X_FFT_KERNELS", "generic")
-        h = PlanewaveHamiltonianApplicator(gpu_context, b)
-        h.update_potential(W.local_potential(c, b, [W.synthetic_species(0)]))
-        try:
-            h.prepare_kpoint(kp)
-        except Exception:
-            if generic:  # the largest planes do not fit the generic kernels
-                break
-            raise
-        out.append((h.apply_batch(psi, FP64), h.apply_batch(psi, MIXED)))
-        if not generic and (kp.fft_map >= 0).all():
-            w = np.array([0.5, 1.0, 2.0])
-            ref = np.zeros(n ** 3)
-            for s in range(3):
-                box = np.zeros(n ** 3, np.complex128)
-                box[kp.fft_map] = psi[:, s]
-                ref += w[s] * np.abs(np.fft.ifftn(box.reshape(n, n, n)).ravel() * box.size) ** 2
-            assert rel_err(h.density(psi, w).ravel(), ref) <= 1e-13
-    if len(out) == 2:
-        assert rel_err(out[0][0], out[1][0]) <= 1e-13
-        assert rel_err(out[0][1], out[1][0]) <= 2e-6
+    v = W.local_potential(c, b, [W.synthetic_species(0)])
+    # plane waves outside the box get the kinetic term only
+    held = np.flatnonzero(kp.fft_map >= 0)
+    w = np.array([0.5, 1.0, 2.0])
+    ref = kp.kinetic_energy_squared[:, None] * psi
+    rho = np.zeros(n ** 3)
+    for s in range(3):
+        box = np.zeros(n ** 3, np.complex128)
+        box[kp.fft_map[held]] = psi[held, s]
+        f = np.fft.ifftn(box.reshape(n, n, n), norm="forward")
+        rho += w[s] * np.abs(f.ravel()) ** 2
+        ref[held, s] += np.fft.fftn(f * np.reshape(v, (n, n, n)), norm="forward").ravel()[kp.fft_map[held]]
+
+    h = PlanewaveHamiltonianApplicator(gpu_context, b)
+    h.update_potential(v)
+    h.prepare_kpoint(kp)
+    assert lib().q3x_debug_plane_form(h.h, FP64) == (2 if inside else 1)
+    assert lib().q3x_debug_plane_form(h.h, MIXED) == (2 if inside else 1)
+    got = h.apply_batch(psi, FP64)
+    assert rel_err(got, ref) <= 1e-13
+    assert rel_err(h.apply_batch(psi, MIXED), ref) <= 2e-6
+    if len(held) == kp.npw:
+        assert rel_err(h.density(psi, w).ravel(), rho) <= 1e-13
+    else:
+        with pytest.raises(Q3XError):
+            h.density(psi, w)
+
+    monkeypatch.setenv("Q3X_FFT_KERNELS", "generic")
+    g = PlanewaveHamiltonianApplicator(gpu_context, b)
+    g.update_potential(v)
+    try:
+        g.prepare_kpoint(kp)
+    except Q3XError as e:
+        assert "does not fit in LDS" in str(e) and n >= 96
+        return
+    assert lib().q3x_debug_plane_form(g.h, FP64) == 0
+    assert rel_err(got, g.apply_batch(psi, FP64)) <= 1e-13
 
 
 def test_sizes_fall_on_both_sides(gpu_context):
