@@ -23,8 +23,9 @@ struct Tile {
 //     and below 0.55 us the copy of the next stage is not either), resident ones overlap,
 //   - each round of resident workgroups costs a prologue and an epilogue, and a split product the
 //     traffic and launch of its reduction.
-// The constants are measured (FP64, one workgroup per CU: 1.06 us a stage at 64 x 64 x 8 against 0.89 of
-// MFMA, 1.31 at 64 x 80 x 8 against 1.12, 0.56 at 32 x 32 x 16 against 0.45).
+// The constants are measured.  A stage with one workgroup on a CU against its share with several, us: FP64
+// 64 x 64 x 8 1.07 / 0.94, 64 x 80 x 8 1.32 / 1.17, 32 x 32 x 16 0.66 / 0.51; FP32 (16 deep) 64 x 64 1.34 / 1.21,
+// 64 x 32 0.91 / 0.69, 32 x 32 0.67 / 0.35, 64 x 16 0.71 / 0.38, for which the model takes 0.55.
 // only: 0, or the one tile to consider; fewest, most: bounds on the number of K chunks.
 struct Choice {
     int tile, split;
