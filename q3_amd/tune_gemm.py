@@ -1,11 +1,11 @@
 """Tile tuner for the complex MFMA GEMM (zgemm64.hip, zgemm32.hip).
 
 Times every tile configuration the library is built with (and a few K splits for the deep-k A^H B
-products; a tile TMWxTNW covers 32 TMW rows and 16 TNW complex columns per workgroup) on the products of H|psi> and block Davidson for a given plane-wave
-count, band count and projector count, and prints the fastest per shape class and precision.
-The library's built-in choices (the cost model of zgemm_split.h)
-were fitted to what this printed for the 64-atom Si cell (npw 51,627, 160 bands, 256 projectors); Q3X_GEMM_TILE="TMWxTNW/ksplit" forces one
-configuration at run time, which is how this script measures the candidates.
+products; a tile TMWxTNW covers 32 TMW rows and 16 TNW complex columns per workgroup) on the products
+of H|psi> and block Davidson for a given plane-wave count, band count and projector count, and prints
+the fastest per shape class and precision beside the library's built-in choice (the cost model of
+zgemm_split.h).  Q3X_GEMM_TILE="TMWxTNW/ksplit" forces one configuration at run time, which is how
+this script measures the candidates.
 
     python -m q3_amd.tune_gemm [--npw 51627] [--bands 160] [--nproj 256] [--reps 20]
 """
@@ -39,7 +39,6 @@ def main(argv=None):
               ("C", 2 * nb, nb, npw, "Gram block"), ("N", npw, nb, 2 * nb, "basis rotation")]
     ctx = Context(0)
     rng = np.random.default_rng(0)
-    warm = True  # the first timings of a fresh process run before the clocks settle
 
     def rnd(shape):
         return np.asfortranarray(rng.standard_normal(shape) + 1j * rng.standard_normal(shape))
@@ -54,14 +53,19 @@ def main(argv=None):
         for prec, label in ((FP64, "fp64"), (MIXED, "fp32")):
             cands = [("", None)] + [(f"{t}/{s}", t) for t in TILES[label] for s in (SPLITS if ta == "C" else [0])]
             best = None
+            # the clocks settle under load: whatever is timed first, the built-in choice, would else look slow
+            os.environ.pop("Q3X_GEMM_TILE", None)
+            t0 = time.perf_counter()
+            while time.perf_counter() - t0 < 0.3:
+                zgemm(ctx, ta, m, n, k, 1.0, A, lda, B, k, 0.0, C, m, prec)
+                ctx.synchronize()
             for cfg, _ in cands:
                 if cfg:
                     os.environ["Q3X_GEMM_TILE"] = cfg
                 else:
                     os.environ.pop("Q3X_GEMM_TILE", None)
-                for _ in range(60 if warm else 3):
+                for _ in range(5):
                     zgemm(ctx, ta, m, n, k, 1.0, A, lda, B, k, 0.0, C, m, prec)
-                warm = False
                 ctx.synchronize()
                 t0 = time.perf_counter()
                 for _ in range(args.reps):
