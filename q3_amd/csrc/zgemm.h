@@ -1,4 +1,4 @@
-// Complex GEMM on MFMA (zgemm.hip).
+// Complex GEMM on MFMA (zgemm.hip, zgemm64.hip, zgemm32.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -7,7 +7,7 @@
 namespace q3x {
 
 // Element types of A, B, the MFMA/accumulation type, and C.  D = complex128, F = complex64.
-enum class GemmTypes { D_D_D_D, F_D_F_F, F_F_F_D, D_D_F_D, F_F_F_F };
+enum class GemmTypes { D_D_D_D, F_D_F_F, F_F_F_D, D_D_F_D };
 
 // C (m x n) = alpha * op(A) * B + beta * C ; opa = 0: A is m x k ; opa = 1: A is k x m, op = A^H.
 // Leading dimensions in complex elements.  work (may be null) enables split-K for skinny shapes.

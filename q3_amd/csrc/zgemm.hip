@@ -13,9 +13,8 @@
 //
 // Workgroup tile: 64 rows x 32 complex columns, or for large FP64 products 128 x 32 or 64 x 80; 4 wave64s
 // in a 2x2 layout; K staged through double-buffered LDS in chunks of 8 complex.
-// Tall-skinny products (k >> m, n: projector overlaps, subspace Gram blocks) split
-// K over the grid's z dimension into a workspace and are summed in a fixed order by a
-// second kernel, so results do not depend on scheduling.
+// Products of few tiles and a long k split K over the grid's z dimension into a workspace and are
+// summed in a fixed order by a second kernel, so results do not depend on scheduling.
 #include <hip/hip_runtime.h>
 
 #include "zgemm.h"
@@ -76,7 +75,7 @@ __global__ void __launch_bounds__(256, MINW) zgemm_kernel(int m, int n, int k, i
     __shared__ TM As[2][2 * KC * LA];
     // FP64 (BC): B stored once per k, row p = [Br Bi Br Bi ...]; row 2p of B' is row p and row
     // 2p + 1 is row p with each (Br, Bi) pair read swapped and its real part negated, which halves
-    // the LDS of B'.  Complex64 keeps B' expanded (its overlap ran 5% slower with the compact form)
+    // the LDS of B'.  FP32 keeps B' expanded (5% faster)
     constexpr bool BC = sizeof(TM) == 8;
     __shared__ TM Bs[2][(BC ? 1 : 2) * KC * LB];
     const int tid = threadIdx.x;
@@ -299,9 +298,8 @@ hipError_t zgemm_shape(int m, int n, int k, double alpha, const void* A, long ld
         ksplit = static_cast<int>(std::max(1L, std::min(want, std::min(by_k, by_ws))));
     }
     // FP64: split K over a multiple of 8 chunks when there are 8 or more, so that each chunk's
-    // tiles share one XCD (xmap in zgemm_kernel).  The complex64 products ran 4% slower with it (1%
-    // with the chunk count kept a multiple of 8: 0.228 vs 0.225 ms for the 256 x 160 x 51,627
-    // overlap) and keep the plain order.
+    // tiles share one XCD (xmap in zgemm_kernel); FP32 products ran 1 to 4% slower with it and keep
+    // the plain order.
     // The chunk count stays that multiple of 8 after the chunk length is rounded up to KC: chunks
     // past the end of K are empty and add zero partials.
     const bool by_xcd = sizeof(TM) == 8 && ksplit >= 8;
@@ -312,9 +310,8 @@ hipError_t zgemm_shape(int m, int n, int k, double alpha, const void* A, long ld
     if (!by_xcd) ksplit = k > 0 ? (k + kchunk - 1) / kchunk : 1;
     int xmap = by_xcd ? 1 : 0;
     dim3 grid(tm, tn, ksplit);
-    // A B without a split (the projector update Hpsi += beta W): the column tiles of a row block
-    // run one after another on one XCD (xmap 2), so each row block of A is fetched once: the
-    // complex64 update of 51,627 x 160 x 256 reads 286 MB instead of 802 MB in the same time
+    // A B without a split: the column tiles of a row block run one after another on one XCD (xmap 2),
+    // so each row block of A is fetched once
     if (OPA == 0 && ksplit == 1 && tn > 1) {
         xmap = 2;
         grid.x = (tm + 7) / 8 * 8;
@@ -388,9 +385,6 @@ hipError_t zgemm(GemmTypes types, int opa, int m, int n, int k, double alpha, co
         case GemmTypes::D_D_F_D:
             return zgemm_t<double, double, float, double>(types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
                                                           work_bytes, st);
-        case GemmTypes::F_F_F_F:
-            return zgemm_t<float, float, float, float>(types, opa, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work,
-                                                       work_bytes, st);
     }
     return hipErrorInvalidValue;
 }
